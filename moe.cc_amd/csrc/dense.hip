@@ -609,88 +609,119 @@ __global__ __launch_bounds__(kRowFinishWaves * kWave) void row_finish_kernel(Den
                    a.sel_p_user ? a.sel_p_user + o : nullptr);
 }
 
-// Many tokens: a block computes a tile of 16*CT tokens x 16*CE rows; thread
-// (ti, ei) owns tokens t0 + ti + 16i and rows n0 + ei + 16j, CT*CE chains.
-// Token and weight rows stream through two LDS chunk buffers of KC columns.
-// Same zero padding and clamping as above.
-template <int CT, int CE, int KC>
-__global__ __launch_bounds__(256) void dense_tile_kernel(DenseArgs a) {
-  constexpr int RX = 16 * CT, RW = 16 * CE, R = RX + RW;
-  constexpr int LD = KC + 4;
-  constexpr int V4 = KC / 4;
-  constexpr int NV = R * V4 / 256;
-  static_assert(R * V4 % 256 == 0, "chunk must split evenly over the block");
-  extern __shared__ float4 lds4[];
-  float* buf = reinterpret_cast<float*>(lds4);   // [2][R][LD]
-  const int tid = threadIdx.x;
-  const int ti = tid / 16, ei = tid % 16;
+// Many tokens, products on the matrix cores: v_mfma_f32_16x16x1_4b with C =
+// 0 and one column per block is four 16 x 16 outer products whose every
+// element is one product x w rounded once, bit for bit v_mul_f32's (checked
+// over random bit patterns, products in and below the denormal range and
+// infinities), so only the adds of the chains are left to the VALU.
+// A wave owns 16 tokens x NB tiles of 16 rows, a block of four waves 16 WX
+// tokens x 16 NB (4 / WX) rows; a lane holds 4 NB chains (tokens 4 (lane /
+// 16) + r, row lane % 16 of each tile).  The four blocks of one MFMA are four
+// columns of one tile: lane (b, i) = (lane / 16, lane % 16) feeds token i and
+// row i of column 4b + c in MFMA c, and result register 4b + r of MFMA c is
+// the product of that column, so the 16 products of a chain's 16 columns are
+// registers of its own lane.  One ds_read_b128 a lane feeds four MFMAs.
+// Operands stream through a D-buffer LDS ring of KC-column chunks with
+// global_load_lds_dwordx4, XOR-swizzled, one barrier a chunk.
+//
+// Bound: VALU issue.  fp32 MFMA and VALU share the fp32 units (a loop of both
+// takes the sum of their times): 2.05 clocks per 64 products and ~2.3 per 64
+// adds with four waves a SIMD, against 4.9 for v_mul_f32 + v_add_f32 whose
+// operand reads also bind on LDS.  Four MFMAs, then their 64 adds: switching
+// between the two costs clocks (4.2 per 64 products in this order, 5.0 with an
+// MFMA before every 16 adds; 6.6 with one wave a SIMD).  512 x 5120 x 2048
+// (the Q/K/V product of a 512-token prompt): 232 -> 172 us; 512 x 2048 x 4096
+// (its O product): 190 -> 156; 100 x 2048 x 4096: 181 -> 60; the add and
+// product floor of the first is 148.
+typedef float v16f __attribute__((ext_vector_type(16)));
+
+__device__ __align__(16) const float kDenseZero[4] = {};
+
+template <int WX, int NB, int KC, int D>
+__global__ __launch_bounds__(256, 4) void dense_mfma_kernel(DenseArgs a) {
+  constexpr int WN = 4 / WX;
+  constexpr int RX = 16 * WX, RW = 16 * NB * WN, R = RX + RW;
+  constexpr int SL = KC / 4;                 // 16-byte slots of an LDS row
+  constexpr int RPI = 64 / SL;               // rows one load instruction covers
+  constexpr int NI = R / RPI;                // load instructions of a chunk
+  constexpr int NL = (NI + 3) / 4;           // per wave
+  static_assert(R % RPI == 0, "whole load instructions");
+  __shared__ float4 lds4[D][R * SL];
+  const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int b = lane / 16, j = lane % 16;
+  const int wx = wave % WX, wn = wave / WX;
   const int t0 = blockIdx.y * RX, n0 = blockIdx.x * RW;
   const int nc = (a.K + KC - 1) / KC;
-  const float* src[NV];
-  int dst[NV], col[NV];
+  // slot s of row r sits at s ^ sw(r): the 16 lanes of one read (rows j, one
+  // slot) then cover all 64 banks
+  auto sw = [](int r) { return KC == 64 ? r & 15 : (r >> 1) & 7; };
+  const float* src[NL];
+  int col[NL];
 #pragma unroll
-  for (int v = 0; v < NV; ++v) {
-    const int i = tid + 256 * v;
-    const int row = i / V4, c4 = i % V4;
-    src[v] = row < RX ? a.A + (size_t)min(t0 + row, a.M - 1) * a.lda + 4 * c4
-                      : a.W + (size_t)min(n0 + row - RX, a.N - 1) * a.ldw + 4 * c4;
-    dst[v] = row * LD + 4 * c4;
-    col[v] = 4 * c4;
+  for (int v = 0; v < NL; ++v) {
+    const int row = RPI * ((wave + 4 * v) % NI) + lane / SL;   // past the tile: another wave's rows again
+    col[v] = 4 * ((lane % SL) ^ sw(row));
+    src[v] = row < RX ? a.A + (size_t)min(t0 + row, a.M - 1) * a.lda + col[v]
+                      : a.W + (size_t)min(n0 + row - RX, a.N - 1) * a.ldw + col[v];
   }
-  float4 rg[NV];
-  auto load = [&](int c) {
+  auto load = [&](int c, int h) {
+    uint8_t* l = reinterpret_cast<uint8_t*>(lds4[h]);
+    if ((c + 1) * KC <= a.K) {
 #pragma unroll
-    for (int v = 0; v < NV; ++v)
-      rg[v] = c * KC + col[v] < a.K ? *reinterpret_cast<const float4*>(src[v] + (size_t)c * KC)
-                                    : zero4();
+      for (int v = 0; v < NL; ++v)
+        lds_load16(src[v] + (size_t)c * KC, l + ((wave + 4 * v) % NI) * 1024);
+    } else {
+#pragma unroll
+      for (int v = 0; v < NL; ++v)
+        lds_load16(c * KC + col[v] < a.K ? src[v] + (size_t)c * KC : kDenseZero,
+                   l + ((wave + 4 * v) % NI) * 1024);
+    }
   };
-  auto store = [&](int b) {
+  float acc[NB][4];
 #pragma unroll
-    for (int v = 0; v < NV; ++v) *reinterpret_cast<float4*>(buf + b * R * LD + dst[v]) = rg[v];
-  };
-  float acc[CT][CE];
+  for (int t = 0; t < NB; ++t)
 #pragma unroll
-  for (int i = 0; i < CT; ++i)
-#pragma unroll
-    for (int j = 0; j < CE; ++j) acc[i][j] = 0.0f;
-  load(0);
-  store(0);
-  if (nc > 1) load(1);
+    for (int r = 0; r < 4; ++r) acc[t][r] = 0.0f;
+  for (int p = 0; p < D - 1; ++p) load(min(p, nc - 1), p);
   for (int c = 0; c < nc; ++c) {
-    __syncthreads();
-    if (c + 1 < nc) {
-      store((c + 1) & 1);
-      if (c + 2 < nc) load(c + 2);
-    }
-    const float* B = buf + (c & 1) * R * LD;
-#pragma unroll 2
-    for (int k = 0; k < KC; k += 4) {
-      float4 xv[CT], wv[CE];
+    stage_sync<(D - 2) * NL>();
+    load(min(c + D - 1, nc - 1), (c + D - 1) % D);
+    const float4* B = lds4[c % D] + j * SL;
+    constexpr int STEPS = KC / 16 * NB;   // 16 columns of one row tile each
+    auto read_x = [&](int g) { return B[16 * wx * SL + ((4 * g + b) ^ sw(j))]; };
+    auto read_w = [&](int t, int g) { return B[(RX + 16 * (NB * wn + t)) * SL + ((4 * g + b) ^ sw(j))]; };
+    float4 x = read_x(0), w = read_w(0, 0);
 #pragma unroll
-      for (int i = 0; i < CT; ++i) xv[i] = *reinterpret_cast<const float4*>(B + (ti + 16 * i) * LD + k);
+    for (int i = 0; i < STEPS; ++i) {
+      const int t = i % NB;
+      float4 xn = x, wn4 = w;
+      if (i + 1 < STEPS) {
+        wn4 = read_w((i + 1) % NB, (i + 1) / NB);
+        if ((i + 1) % NB == 0) xn = read_x((i + 1) / NB);
+      }
+      asm volatile("" ::: "memory");   // the next step's operands are requested here, not sunk to their use
+      v16f p[4];
+      p[0] = __builtin_amdgcn_mfma_f32_16x16x1f32(x.x, w.x, v16f{}, 0, 0, 0);
+      p[1] = __builtin_amdgcn_mfma_f32_16x16x1f32(x.y, w.y, v16f{}, 0, 0, 0);
+      p[2] = __builtin_amdgcn_mfma_f32_16x16x1f32(x.z, w.z, v16f{}, 0, 0, 0);
+      p[3] = __builtin_amdgcn_mfma_f32_16x16x1f32(x.w, w.w, v16f{}, 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int j = 0; j < CE; ++j) wv[j] = *reinterpret_cast<const float4*>(B + (RX + ei + 16 * j) * LD + k);
+      for (int k = 0; k < 16; ++k)
 #pragma unroll
-      for (int i = 0; i < CT; ++i)
-#pragma unroll
-        for (int j = 0; j < CE; ++j) {
-          const float p0 = xv[i].x * wv[j].x, p1 = xv[i].y * wv[j].y;
-          const float p2 = xv[i].z * wv[j].z, p3 = xv[i].w * wv[j].w;
-          float s = acc[i][j];
-          s = s + p0;
-          s = s + p1;
-          s = s + p2;
-          s = s + p3;
-          acc[i][j] = s;
-        }
+        for (int r = 0; r < 4; ++r) acc[t][r] = acc[t][r] + p[k % 4][4 * (k / 4) + r];
+      __builtin_amdgcn_sched_barrier(0);
+      x = xn;
+      w = wn4;
     }
   }
+  stage_sync<0>();   // the clamped loads past the last chunk have landed
 #pragma unroll
-  for (int i = 0; i < CT; ++i)
+  for (int t = 0; t < NB; ++t)
 #pragma unroll
-    for (int j = 0; j < CE; ++j) {
-      const int t = t0 + ti + 16 * i, n = n0 + ei + 16 * j;
-      if (t < a.M && n < a.N) a.C[(size_t)t * a.ldc + n] = dense_epilogue(a, t, n, acc[i][j]);
+    for (int r = 0; r < 4; ++r) {
+      const int tok = t0 + 16 * wx + 4 * b + r, n = n0 + 16 * (NB * wn + t) + j;
+      if (tok < a.M && n < a.N) a.C[(size_t)tok * a.ldc + n] = dense_epilogue(a, tok, n, acc[t][r]);
     }
 }
 
@@ -1524,6 +1555,42 @@ moe_status set_lds(F* fn, size_t bytes, const char* what) {
   return st;
 }
 
+template <int WX, int NB, int KC, int D>
+moe_status launch_mfma(const DenseArgs& a, hipStream_t s) {
+  constexpr int RX = 16 * WX, RW = 16 * NB * (4 / WX);
+  dim3 grid((unsigned)((a.N + RW - 1) / RW), (unsigned)((a.M + RX - 1) / RX));
+  hipLaunchKernelGGL((dense_mfma_kernel<WX, NB, KC, D>), grid, dim3(256), 0, s, a);
+  return check_hip(hipGetLastError(), "dense mfma launch");
+}
+
+// The tile shape with the least estimated time.  Per column of K a CU with m
+// blocks takes about step * m clocks, and `odd` more when m is odd (a SIMD's
+// last wave runs alone: 6.6 clocks per 64 products against 4.5 for two).
+// Measured, clocks per column at K = 2048 and 4096: 32 x 32 tiles 37, 55, 73,
+// 88, 234 for m = 1, 2, 3, 4, 10; 32 x 64 65, 91, 131, 210 for m = 1, 2, 3, 5;
+// 64 x 64 116, 160, 246, 586 for m = 1, 2, 3, 8; 64 x 80 145, 199, 305 for m =
+// 1, 2, 3.  Small tiles spread few tokens over the CUs, large ones spend less
+// on operands per product.
+moe_status launch_mfma_best(const DenseArgs& a, hipStream_t s) {
+  struct Shape { int rx, rw, step, odd; };
+  static const Shape shapes[4] = {{32, 32, 22, 10}, {32, 64, 40, 18}, {64, 64, 75, 42}, {64, 80, 95, 50}};
+  int best = 0;
+  double tbest = 0.0;
+  for (int i = 0; i < 4; ++i) {
+    const Shape& h = shapes[i];
+    const long long blocks = (long long)((a.N + h.rw - 1) / h.rw) * ((a.M + h.rx - 1) / h.rx);
+    const long long m = (blocks + 255) / 256;
+    const double t = (double)m * h.step + (m & 1) * h.odd;
+    if (i == 0 || t < tbest) { best = i; tbest = t; }
+  }
+  switch (best) {
+    case 0: return launch_mfma<2, 1, 64, 2>(a, s);
+    case 1: return launch_mfma<2, 2, 32, 2>(a, s);
+    case 2: return launch_mfma<4, 4, 32, 2>(a, s);
+    default: return launch_mfma<4, 5, 32, 2>(a, s);
+  }
+}
+
 size_t gemv_lds(int RW, int NP, int M, int K, bool norm) {
   const int KC = RW >= 16 ? 4096 / RW : 256;
   return ((size_t)(NP + 1) * M * RW * (KC + 4) + (norm ? (size_t)M * K : 0)) * 4;
@@ -1537,14 +1604,6 @@ moe_status launch_gemv(const DenseArgs& a, hipStream_t s) {
   hipLaunchKernelGGL((dense_gemv_kernel<RW, NORM, PACK, NP, MMX>), dim3((unsigned)((a.N + RW - 1) / RW)),
                      dim3(64 * (NP + 1)), lds, s, a);
   return check_hip(hipGetLastError(), "dense gemv launch");
-}
-
-template <int CT, int CE, int KC>
-moe_status launch_tile(const DenseArgs& a, hipStream_t s) {
-  constexpr size_t lds = 2 * (size_t)(16 * CT + 16 * CE) * (KC + 4) * 4;
-  dim3 grid((unsigned)((a.N + 16 * CE - 1) / (16 * CE)), (unsigned)((a.M + 16 * CT - 1) / (16 * CT)));
-  hipLaunchKernelGGL((dense_tile_kernel<CT, CE, KC>), grid, dim3(256), lds, s, a);
-  return check_hip(hipGetLastError(), "dense tile launch");
 }
 
 }  // namespace
@@ -1706,19 +1765,15 @@ moe_status dense_matmul(const DenseArgs& a, hipStream_t s) {
     return launch_gemv<8, false, 0, kNpOne, 1>(a, s);
   } else if (a.M <= 4) {
     return launch_gemv<16, false, 0, 1>(a, s);
-  } else if (a.M <= 16) {
+  } else if (a.M <= 8 && (long long)a.M * a.N < 40000) {
+    // the chain kernel costs ~6 us per 1024 rows at M = 8, K = 2048, the MFMA
+    // tiles 30 us up to 8192 rows: 22 against 30 us at 5 x 5120, 35 against
+    // 30 at 8 x 5120, 23 against 57 at 8 x 2048 x 4096; from 9 tokens the
+    // tiles are never slower (16 x 1100 x 1024: 21 against 16)
     return launch_gemv<4, false, 0, 1>(a, s);
-  } else if (a.M >= 256 && (long long)((a.N + 63) / 64) * ((a.M + 63) / 64) >= 1024) {
-    // 64 x 64 tiles only with >= 1024 blocks; below that 32-token x 64-row
-    // tiles keep more waves on each SIMD (prefill at T = 512: Wo 256 and
-    // [Wq;Wk;Wv] 640 blocks of 64 x 64; the model's 512-token prefill 49.7
-    // -> 43.5 ms with 32 x 32 tiles, 41.5 -> 39.8 ms with 32 x 64: eight
-    // chains a thread, each x value read for four rows)
-    return launch_tile<4, 4, 32>(a, s);
   } else {
-    return launch_tile<2, 4, 64>(a, s);
+    return launch_mfma_best(a, s);
   }
-  return check_hip(hipGetLastError(), "dense gemv launch");
 }
 
 moe_status embed_rows(const int32_t* ids, int T, const float* emb, int V, int D, float* x,

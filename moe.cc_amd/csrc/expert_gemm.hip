@@ -151,22 +151,6 @@ struct EgCfg {
   static_assert(NP <= kEgPairs, "pairs of a pass");
 };
 
-// One 16-byte-per-lane global -> LDS load: lane i's 16 bytes from src land at
-// LDS address lds + 16 i.  Issued from inline asm so that the compiler's
-// wait-count bookkeeping, which does not place these loads correctly among
-// the register loads, never sees them: every wait for them is explicit
-// (stage_sync), and the compiler's own vmcnt waits only grow stricter.
-// M0 is reserved to the compiler, which uses it in these kernels for nothing
-// else (checked in the generated code), so setting it here is safe.
-__device__ __forceinline__ void lds_load16(const void* src, uint8_t* lds) {
-  const uint32_t la = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)lds);
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(la)
-               : "memory", "m0");
-#pragma clang diagnostic pop
-}
-
 // Sixteen zero bytes: the B source of an h-table unit whose segment's values
 // needed fewer limbs than the pass's limb (the gate/up epilogue writes only
 // the planes a segment needs).
@@ -243,15 +227,6 @@ __device__ __forceinline__ void stage_load(const EgSrc<Q4, C>& src, int st, size
     }
     lds_load16(b, buf + C::W_BYTES + ins * 1024);
   }
-}
-
-// Waits for this wave's loads of the stage about to be read (N later loads
-// may stay in flight) and its LDS reads, then joins the block: after it the
-// whole stage is in LDS and every wave is done with the buffer that the
-// next loads overwrite.
-template <int N>
-__device__ __forceinline__ void stage_sync() {
-  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
 }
 
 // stage_sync with N = (D - 2) q, q this wave's loads per stage (uniform).

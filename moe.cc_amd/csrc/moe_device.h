@@ -381,4 +381,29 @@ __device__ __forceinline__ float silu_mul_t(float g, float u, const uint64_t* ta
 }
 __device__ __forceinline__ float silu_mul(float g, float u) { return silu_mul_t(g, u, kExp2Tab); }
 
+// One 16-byte-per-lane global -> LDS load: lane i's 16 bytes from src land at
+// LDS address lds + 16 i.  Issued from inline asm so that the compiler's
+// wait-count bookkeeping, which does not place these loads correctly among
+// the register loads, never sees them: every wait for them is explicit
+// (stage_sync), and the compiler's own vmcnt waits only grow
+// stricter.  M0 is reserved to the compiler, which uses it in these kernels
+// for nothing else (checked in the generated code), so setting it here is
+// safe.
+__device__ __forceinline__ void lds_load16(const void* src, uint8_t* lds) {
+  const uint32_t la = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)lds);
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(la)
+               : "memory", "m0");
+#pragma clang diagnostic pop
+}
+
+// Waits for this wave's lds_load16 loads but the N last ones and for its LDS
+// reads, then joins the block: after it every wave's loads up to there are in
+// LDS and every wave is done with the buffer that the next loads overwrite.
+template <int N>
+__device__ __forceinline__ void stage_sync() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
+}
+
 }  // namespace moe
