@@ -41,6 +41,7 @@
 // the 8 even columns then the 8 odd ones (the order a packed weight dword's
 // low nibbles, then high nibbles, take).  The router blocks write the x
 // tables (pack_unit16, moe_grouped.hip), the gate/up epilogue the h tables.
+#include <algorithm>
 #include <utility>
 
 #include "moe_device.h"
@@ -169,7 +170,7 @@ struct EgSrc {
   int col[C::PERB];         // column of this lane's B unit within a stage
 };
 
-template <bool Q4, class C, class WRow>
+template <bool Q4, class C, int LP, class WRow>
 __device__ __forceinline__ void eg_sources(EgSrc<Q4, C>& src, WRow&& wrow, const EgPairs& sp,
                                            int pbase, int n, int K, int l, const uint32_t* segmask) {
   using SG = EgStage<Q4>;
@@ -184,9 +185,10 @@ __device__ __forceinline__ void eg_sources(EgSrc<Q4, C>& src, WRow&& wrow, const
     const int ins = (wave + C::W * k) % C::NIB;
     const int row = ins * SG::RPI + lane / SG::UNITS;
     const int unit = (lane % SG::UNITS) ^ swz<Q4>(row);
-    const int q = min(pbase + row, n - 1);
-    src.b[k] = reinterpret_cast<const uint8_t*>(act_plane(sp.tab[q], K, l)) + unit * 16;
-    src.segs[k] = segmask && l > 0 ? segmask[(l - 1) * kEgPairs + q] : ~0u;
+    const int t = row / 32 / C::PG, lr = l + t % LP;   // B tile of the wave's pair group, its limb
+    const int q = min(pbase + 32 * (t / LP * C::PG + row / 32 % C::PG) + row % 32, n - 1);
+    src.b[k] = reinterpret_cast<const uint8_t*>(act_plane(sp.tab[q], K, lr)) + unit * 16;
+    src.segs[k] = segmask && lr > 0 ? segmask[(lr - 1) * kEgPairs + q] : ~0u;
     src.col[k] = unit * 16;
   }
   // B instructions past the pass's pairs are not issued (shapes of more
@@ -194,7 +196,8 @@ __device__ __forceinline__ void eg_sources(EgSrc<Q4, C>& src, WRow&& wrow, const
   // measured faster with every wave issuing PERB): instruction ins holds
   // pair rows ins * RPI ..; this wave issues ins = wave + W k
   if constexpr (C::NP > 128) {
-    const int live = min(n - pbase, C::NP);
+    int live = min(n - pbase, C::NP / LP);
+    if constexpr (LP > 1) live = (live + 32 * C::PG - 1) / (32 * C::PG) * (32 * C::PG) * LP;
     const int nins = (live + SG::RPI - 1) / SG::RPI;
     src.nb = __builtin_amdgcn_readfirstlane(min(max((nins - wave + C::W - 1) / C::W, 0), C::PERB));
   } else {
@@ -256,8 +259,8 @@ __device__ __forceinline__ WFrag32 w_frag(const uint8_t* wbuf, int m) {
 
 // One step of the stage ring: wait for the stage in buffer cbuf, issue the
 // loads of K stage lst (weights woff bytes further) into buffer lbuf, then
-// the MFMAs of buffer cbuf: acc[m][t] for this wave's live pair tiles t <
-// NL.
+// the MFMAs of buffer cbuf: acc[m][t] for this wave's live B tiles t < NL
+// (a pair tile has LP of them, one a limb).
 template <bool Q4, int RG, int NTW, int D, int NW, int NL, bool SEGM>
 __device__ __forceinline__ void eg_stage(const EgSrc<Q4, EgCfg<Q4, RG, NTW, D, NW>>& src, int lst,
                                          size_t woff, int lbuf, int cbuf, uint8_t* lds,
@@ -310,14 +313,14 @@ __device__ __forceinline__ void eg_stage(const EgSrc<Q4, EgCfg<Q4, RG, NTW, D, N
   }
 }
 
-// The stage loop of a wave with NL live tiles; NL is chosen once per pass
+// The stage loop of a wave with NL live B tiles; NL is chosen once per pass
 // (live_tiles), so that the MFMA sequence of a stage has no branches.
-template <bool Q4, int RG, int NTW, int D, int NW, int NL, bool SEGM>
+template <bool Q4, int RG, int NTW, int D, int NW, int NL, int LP, bool SEGM>
 __device__ __forceinline__ void eg_loop(const EgSrc<Q4, EgCfg<Q4, RG, NTW, D, NW>>& src, int nst, int rot,
                                         int ntl, uint8_t* lds, v16i (&acc)[2][NTW]) {
   if constexpr (NL > 0) {
     if (ntl < NL) {
-      eg_loop<Q4, RG, NTW, D, NW, NL - 1, SEGM>(src, nst, rot, ntl, lds, acc);
+      eg_loop<Q4, RG, NTW, D, NW, NL - LP, LP, SEGM>(src, nst, rot, ntl, lds, acc);
       return;
     }
   }
@@ -330,17 +333,18 @@ __device__ __forceinline__ void eg_loop(const EgSrc<Q4, EgCfg<Q4, RG, NTW, D, NW
 // apart): step g is K stage g % nst of row tile g / nst, so the first loads
 // of a tile are issued during the last stages of the one before.  After a
 // tile's last stage epi(r, acc) takes its dots (epi must leave the ring
-// alone) and the accumulators restart.  One limb (no segment masks).
-template <bool Q4, int RG, int NTW, int D, int NW, int NL, class Epi>
+// alone) and the accumulators restart.  All limbs in one pass.
+template <bool Q4, int RG, int NTW, int D, int NW, int NL, int LP, class Epi>
 __device__ __forceinline__ void eg_loop_rows(const EgSrc<Q4, EgCfg<Q4, RG, NTW, D, NW>>& src, int nst,
                                              int rot, int R, size_t wstep, int ntl, uint8_t* lds, Epi& epi) {
   if constexpr (NL > 0) {
     if (ntl < NL) {
-      eg_loop_rows<Q4, RG, NTW, D, NW, NL - 1>(src, nst, rot, R, wstep, ntl, lds, epi);
+      eg_loop_rows<Q4, RG, NTW, D, NW, NL - LP, LP>(src, nst, rot, R, wstep, ntl, lds, epi);
       return;
     }
   }
   using C = EgCfg<Q4, RG, NTW, D, NW>;
+  constexpr bool SEGM = LP > 1;   // planes past a segment's limbs read as zeros
   v16i acc[2][NTW];
 #pragma unroll
   for (int m = 0; m < 2; ++m)
@@ -349,12 +353,12 @@ __device__ __forceinline__ void eg_loop_rows(const EgSrc<Q4, EgCfg<Q4, RG, NTW, 
   const int total = nst * R;
   for (int p = 0; p < D - 1; ++p) {
     const int gl = min(p, total - 1);
-    stage_load<Q4, C, false, 32 * RG>(src, (gl % nst + rot) % nst, (size_t)(gl / nst) * wstep,
+    stage_load<Q4, C, SEGM, 32 * RG>(src, (gl % nst + rot) % nst, (size_t)(gl / nst) * wstep,
                                       lds + p * C::STAGE);
   }
   for (int g = 0; g < total; ++g) {
     const int gl = min(g + D - 1, total - 1);
-    eg_stage<Q4, RG, NTW, D, NW, NL, false>(src, (gl % nst + rot) % nst, (size_t)(gl / nst) * wstep,
+    eg_stage<Q4, RG, NTW, D, NW, NL, SEGM>(src, (gl % nst + rot) % nst, (size_t)(gl / nst) * wstep,
                                             (g + D - 1) % D, g % D, lds, acc);
     if (g % nst == nst - 1) {
       epi(g / nst, acc);
@@ -368,7 +372,8 @@ __device__ __forceinline__ void eg_loop_rows(const EgSrc<Q4, EgCfg<Q4, RG, NTW, 
 }
 
 // Live pair tiles of this wave in a pass over pairs pbase .. n - 1: tiles t
-// with 32 (t PG + pg) < n - pbase.  The same for every lane of the wave.
+// with 32 (t PG + pg) < n - pbase, at most NTW.  The same for every lane of
+// the wave.
 template <int PG, int NTW>
 __device__ __forceinline__ int live_tiles(int pbase, int n, int pg) {
   const int live = n - pbase;   // >= 1
@@ -377,23 +382,23 @@ __device__ __forceinline__ int live_tiles(int pbase, int n, int pg) {
   return __builtin_amdgcn_readfirstlane(min(max(t, 0), NTW));
 }
 
-// acc[m][t] = sum over all K columns of W_m[lane's row] x limb l of pair
-// pbase + 32 (NTW pg + t) + (lane % 32).  Every thread of the block calls
+// acc[m][LP t + i] = sum over all K columns of W_m[lane's row] x limb l + i of
+// pair pbase + 32 (PG t + pg) + (lane % 32).  Every thread of the block calls
 // this.  On return every load of the pass has landed and every wave is done
 // with the LDS ring.
-template <bool Q4, int RG, int NTW, int D, int NW, bool SEGM, class WRow>
+template <bool Q4, int RG, int NTW, int D, int NW, int LP, bool SEGM, class WRow>
 __device__ __forceinline__ void eg_pass(WRow&& wrow, int K, const EgPairs& sp, int pbase, int n,
                                         int l, const uint32_t* segmask, uint8_t* lds, v16i (&acc)[2][NTW]) {
   using SG = EgStage<Q4>;
   using C = EgCfg<Q4, RG, NTW, D, NW>;
   const int nst = K / SG::COLS;
-  const int ntl = live_tiles<C::PG, NTW>(pbase, n, (threadIdx.x / kWave) / RG);
+  const int ntl = LP * live_tiles<C::PG, NTW / LP>(pbase, n, (threadIdx.x / kWave) / RG);
 #pragma unroll
   for (int m = 0; m < 2; ++m)
 #pragma unroll
     for (int t = 0; t < NTW; ++t) acc[m][t] = v16i{};
   EgSrc<Q4, C> src;
-  eg_sources<Q4, C>(src, wrow, sp, pbase, n, K, l, segmask);
+  eg_sources<Q4, C, LP>(src, wrow, sp, pbase, n, K, l, segmask);
   // the stages run in a rotated order, one per task (the dots are exact in
   // any order): concurrent tasks read different column slices of their
   // rows, while the row blocks of one task (one XCD, dispatched together)
@@ -403,51 +408,79 @@ __device__ __forceinline__ void eg_pass(WRow&& wrow, int K, const EgPairs& sp, i
 #pragma unroll
   for (int p = 0; p < D - 1; ++p)
     stage_load<Q4, C, SEGM, 32 * RG>(src, (min(p, nst - 1) + rot) % nst, 0, lds + p * C::STAGE);
-  eg_loop<Q4, RG, NTW, D, NW, NTW, SEGM>(src, nst, rot, ntl, lds, acc);
+  eg_loop<Q4, RG, NTW, D, NW, NTW, LP, SEGM>(src, nst, rot, ntl, lds, acc);
   // the clamped loads past the last stage land before the ring is reused
   stage_sync<0>();
 }
 
-// Dots of a pass over all limbs: one pass (nl == 1) or limb passes folded
-// into wrapping uint32 totals.  segmask (down: [3][kEgPairs] in LDS, else
-// null): bit s of segmask[l - 1][pair] says segment s of the pair's h
-// table holds limb plane l.
-template <bool Q4, int RG, int NTW, int D, int NW, class WRow>
+// The dots of pair tile t from the accumulators of its limbs l .. l + LP - 1,
+// folded into wrapping uint32 totals.
+template <int LP, int NTW>
+__device__ __forceinline__ v16u fold_limbs(const v16i (&acc)[NTW], int t, int l) {
+  v16u d = __builtin_bit_cast(v16u, acc[LP * t]) << (8u * l);
+#pragma unroll
+  for (int i = 1; i < LP; ++i) d += __builtin_bit_cast(v16u, acc[LP * t + i]) << (8u * (l + i));
+  return d;
+}
+
+// Dots of pairs pbase .. over all limbs: one pass for up to LP limbs, else
+// one per LP limbs.  Two limbs a pass read the weights once for both (a pass
+// per limb streamed them from HBM again: gate/up of 300 tokens, Q8, 2-limb
+// activations, 137 -> 87 us; down 75 -> 52).  segmask (down: [3][kEgPairs] in LDS, else
+// null): bit s of segmask[l - 1][pair] says segment s of the pair's h table
+// holds limb plane l.
+template <bool Q4, int RG, int NTW, int D, int NW, int LP, class WRow>
 __device__ __forceinline__ void eg_dots(WRow&& wrow, int K, const EgPairs& sp, int pbase, int n,
                                         int nl, const uint32_t* segmask, uint8_t* lds,
-                                        v16u (&dots)[2][NTW]) {
+                                        v16u (&dots)[2][NTW / LP]) {
   v16i acc[2][NTW];
-  eg_pass<Q4, RG, NTW, D, NW, false>(wrow, K, sp, pbase, n, 0, nullptr, lds, acc);
-#pragma unroll
-  for (int m = 0; m < 2; ++m)
-#pragma unroll
-    for (int t = 0; t < NTW; ++t) dots[m][t] = __builtin_bit_cast(v16u, acc[m][t]);
-  for (int l = 1; l < nl; ++l) {
-    if (segmask)
-      eg_pass<Q4, RG, NTW, D, NW, true>(wrow, K, sp, pbase, n, l, segmask, lds, acc);
+  for (int l = 0; l < nl; l += LP) {
+    if (segmask && l + LP > 1)
+      eg_pass<Q4, RG, NTW, D, NW, LP, true>(wrow, K, sp, pbase, n, l, segmask, lds, acc);
     else
-      eg_pass<Q4, RG, NTW, D, NW, false>(wrow, K, sp, pbase, n, l, nullptr, lds, acc);
+      eg_pass<Q4, RG, NTW, D, NW, LP, false>(wrow, K, sp, pbase, n, l, nullptr, lds, acc);
 #pragma unroll
     for (int m = 0; m < 2; ++m)
 #pragma unroll
-      for (int t = 0; t < NTW; ++t) dots[m][t] += __builtin_bit_cast(v16u, acc[m][t]) << (8u * l);
+      for (int t = 0; t < NTW / LP; ++t) {
+        const v16u d = fold_limbs<LP>(acc[m], t, l);
+        dots[m][t] = l == 0 ? d : dots[m][t] + d;
+      }
   }
 }
 
-// One-limb dots of R consecutive row tiles (weights wstep bytes apart) over
-// all n pairs of the task, epi(r, acc) after each tile (eg_loop_rows).
-template <bool Q4, int RG, int NTW, int D, int NW, class WRow, class Epi>
+// Dots (at most LP limbs) of R consecutive row tiles (weights wstep bytes
+// apart) over all n pairs of the task, epi(r, acc) after each tile
+// (eg_loop_rows).
+template <bool Q4, int RG, int NTW, int D, int NW, int LP, class WRow, class Epi>
 __device__ __forceinline__ void eg_rows(WRow&& wrow, int K, const EgPairs& sp, int n, int R, size_t wstep,
-                                        uint8_t* lds, Epi&& epi) {
+                                        const uint32_t* segmask, uint8_t* lds, Epi&& epi) {
   using SG = EgStage<Q4>;
   using C = EgCfg<Q4, RG, NTW, D, NW>;
   const int nst = K / SG::COLS;
-  const int ntl = live_tiles<C::PG, NTW>(0, n, (threadIdx.x / kWave) / RG);
+  const int ntl = LP * live_tiles<C::PG, NTW / LP>(0, n, (threadIdx.x / kWave) / RG);
   EgSrc<Q4, C> src;
-  eg_sources<Q4, C>(src, wrow, sp, 0, n, K, 0, nullptr);
+  eg_sources<Q4, C, LP>(src, wrow, sp, 0, n, K, 0, segmask);
   const int rot = sp.rot % nst;
-  eg_loop_rows<Q4, RG, NTW, D, NW, NTW>(src, nst, rot, R, wstep, ntl, lds, epi);
+  eg_loop_rows<Q4, RG, NTW, D, NW, NTW, LP>(src, nst, rot, R, wstep, ntl, lds, epi);
 }
+
+// Shape of the passes over tasks with multi-limb activations.  Q8 (nearly
+// every task: |x| > 1 needs two limbs): two limbs a pass, so that the B tiles
+// hold half as many pairs as with one (one pair tile a wave at least), and a
+// ring stage less where it would not fit beside another block's.  Q4 (|x| >
+// 18): a pass per limb over half the pairs; the two-limb code cost its
+// one-limb tasks 2-4% in registers and LDS.
+template <bool Q4, int RG, int NTW, int D, int NW>
+struct EgMulti {
+  using C1 = EgCfg<Q4, RG, NTW, D, NW>;
+  static constexpr int LP = Q4 ? 1 : 2;                        // limbs of a pass
+  static constexpr int NT = Q4 ? (NTW > 1 ? NTW / 2 : 1) : (NTW > 1 ? NTW : 2);   // B tiles a wave
+  static constexpr int DL = EgCfg<Q4, RG, NT, D, NW>::BYTES <= C1::BYTES + 12 * 1024 ? D : D - 1;
+  using C = EgCfg<Q4, RG, NT, DL, NW>;
+  static constexpr int PT = NT / LP;                           // pair tiles a wave
+  static constexpr int NP = C::NP / LP;                        // pairs of a pass
+};
 
 // Where row r of an activation unit table sits in its limb plane.
 template <bool Q4>
@@ -667,22 +700,23 @@ __global__ __launch_bounds__(64 * NW) void gate_up_eg_kernel(EgArgs a) {
   };
   const int nlt = sp.nl;
   // half the tiles and one more ring stage (DH) when they fit the same LDS:
-  // the 256-pair shape's tasks of at most 128 pairs, and its limb passes
+  // the 256-pair shape's tasks of at most 128 pairs
   constexpr int NTM = NTW > 1 ? NTW / 2 : 1;
   constexpr int DH = EgCfg<Q4, RG, NTM, D + 1, NW>::BYTES <= C::BYTES && C::NP > 128 ? D + 1 : D;
   if (nlt == 1 && (DH == D || n > EgCfg<Q4, RG, NTM, DH, NW>::NP)) {
     v16u dots[2][NTW];
-    eg_dots<Q4, RG, NTW, D, NW>(wrow, a.K, sp, 0, n, 1, nullptr, lds, dots);
+    eg_dots<Q4, RG, NTW, D, NW, 1>(wrow, a.K, sp, 0, n, 1, nullptr, lds, dots);
     gate_up_epi<Q4, RG, C::PG, NTW, C::BYTES>(a, sp, dots, 0, n, rb, sg, su, exp_tab, lds, &multi_flag);
-  } else {
-    // limb passes over half as many pairs at a time (the totals take the
-    // other half of the accumulator budget); one limb here when the task
-    // fits a half pass
-    constexpr int NPM = EgCfg<Q4, RG, NTM, DH, NW>::NP;
+  } else if (nlt == 1) {
     v16u dots[2][NTM];
-    for (int pb = 0; pb < n; pb += NPM) {
-      eg_dots<Q4, RG, NTM, DH, NW>(wrow, a.K, sp, pb, n, nlt, nullptr, lds, dots);
-      gate_up_epi<Q4, RG, C::PG, NTM, C::BYTES>(a, sp, dots, pb, n, rb, sg, su, exp_tab, lds, &multi_flag);
+    eg_dots<Q4, RG, NTM, DH, NW, 1>(wrow, a.K, sp, 0, n, 1, nullptr, lds, dots);
+    gate_up_epi<Q4, RG, C::PG, NTM, C::BYTES>(a, sp, dots, 0, n, rb, sg, su, exp_tab, lds, &multi_flag);
+  } else {
+    using X = EgMulti<Q4, RG, NTW, D, NW>;
+    v16u dots[2][X::PT];
+    for (int pb = 0; pb < n; pb += X::NP) {
+      eg_dots<Q4, RG, X::NT, X::DL, NW, X::LP>(wrow, a.K, sp, pb, n, nlt, nullptr, lds, dots);
+      gate_up_epi<Q4, RG, C::PG, X::PT, C::BYTES>(a, sp, dots, pb, n, rb, sg, su, exp_tab, lds, &multi_flag);
     }
   }
   __syncthreads();
@@ -830,7 +864,7 @@ __global__ __launch_bounds__(64 * NW) void down_eg_kernel(EgArgs a) {
         for (int q = 0; q < NTW; ++q) dots[m][q] = __builtin_bit_cast(v16u, acc[m][q]);
       down_epi<Q4, RG, C::PG, NTW>(a, sp, dots, 0, n, rb0 + t * BR, sd + t * BR);
     };
-    eg_rows<Q4, RG, NTW, D, NW>(wrow, a.K, sp, n, R, (size_t)BR * a.rb, lds, epi);
+    eg_rows<Q4, RG, NTW, D, NW, 1>(wrow, a.K, sp, n, R, (size_t)BR * a.rb, nullptr, lds, epi);
   } else if (nlt == 1) {
     auto epi = [&](int t, v16i (&acc)[2][NTM]) {
       v16u dots[2][NTM];
@@ -840,16 +874,29 @@ __global__ __launch_bounds__(64 * NW) void down_eg_kernel(EgArgs a) {
         for (int q = 0; q < NTM; ++q) dots[m][q] = __builtin_bit_cast(v16u, acc[m][q]);
       down_epi<Q4, RG, C::PG, NTM>(a, sp, dots, 0, n, rb0 + t * BR, sd + t * BR);
     };
-    eg_rows<Q4, RG, NTM, DH, NW>(wrow, a.K, sp, n, R, (size_t)BR * a.rb, lds, epi);
+    eg_rows<Q4, RG, NTM, DH, NW, 1>(wrow, a.K, sp, n, R, (size_t)BR * a.rb, nullptr, lds, epi);
+  } else if (nlt == 2 && EgMulti<Q4, RG, NTW, D, NW>::LP == 2 && n <= EgMulti<Q4, RG, NTW, D, NW>::NP) {
+    using X = EgMulti<false, RG, NTW, D, NW>;   // (Q8)
+    if constexpr (!Q4) {
+      auto epi = [&](int t, v16i (&acc)[2][X::NT]) {
+        v16u dots[2][X::PT];
+#pragma unroll
+        for (int m = 0; m < 2; ++m)
+#pragma unroll
+          for (int q = 0; q < X::PT; ++q) dots[m][q] = fold_limbs<2>(acc[m], q, 0);
+        down_epi<Q4, RG, C::PG, X::PT>(a, sp, dots, 0, n, rb0 + t * BR, sd + t * BR);
+      };
+      eg_rows<Q4, RG, X::NT, X::DL, NW, 2>(wrow, a.K, sp, n, R, (size_t)BR * a.rb, segmask, lds, epi);
+    }
   } else {
-    constexpr int NPM = EgCfg<Q4, RG, NTM, DH, NW>::NP;
-    v16u dots[2][NTM];
+    using X = EgMulti<Q4, RG, NTW, D, NW>;
+    v16u dots[2][X::PT];
     for (int t = 0; t < R; ++t) {
       const int rb = rb0 + t * BR;
       auto wrow_t = [&](int r) { return w0 + (size_t)min(rb + r, a.rows - 1) * a.rb; };
-      for (int pb = 0; pb < n; pb += NPM) {
-        eg_dots<Q4, RG, NTM, DH, NW>(wrow_t, a.K, sp, pb, n, nlt, segmask, lds, dots);
-        down_epi<Q4, RG, C::PG, NTM>(a, sp, dots, pb, n, rb, sd + t * BR);
+      for (int pb = 0; pb < n; pb += X::NP) {
+        eg_dots<Q4, RG, X::NT, X::DL, NW, X::LP>(wrow_t, a.K, sp, pb, n, nlt, segmask, lds, dots);
+        down_epi<Q4, RG, C::PG, X::PT>(a, sp, dots, pb, n, rb, sd + t * BR);
       }
     }
   }
@@ -874,10 +921,11 @@ template <bool Q4, int RG, int NTW, int D, int NW, int RTPB>
 moe_status launch_eg_shape(const LayerDev* L, int ntask, hipStream_t s) {
   static_assert(RTPB >= 1 && RTPB <= kDownRowTiles, "down row tiles per block");
   using C = EgCfg<Q4, RG, NTW, D, NW>;
+  constexpr size_t lds = std::max(C::BYTES, EgMulti<Q4, RG, NTW, D, NW>::C::BYTES);
   static bool attr = false;
-  if (!attr && C::BYTES > 65536) {
-    moe_status st = eg_lds_attr(gate_up_eg_kernel<Q4, RG, NTW, D, NW>, C::BYTES, "expert gate/up LDS attribute");
-    if (!st) st = eg_lds_attr(down_eg_kernel<Q4, RG, NTW, D, NW>, C::BYTES, "expert down LDS attribute");
+  if (!attr && lds > 65536) {
+    moe_status st = eg_lds_attr(gate_up_eg_kernel<Q4, RG, NTW, D, NW>, lds, "expert gate/up LDS attribute");
+    if (!st) st = eg_lds_attr(down_eg_kernel<Q4, RG, NTW, D, NW>, lds, "expert down LDS attribute");
     if (st) return st;
     attr = true;
   }
@@ -887,7 +935,7 @@ moe_status launch_eg_shape(const LayerDev* L, int ntask, hipStream_t s) {
            L->xtab, act_table_bytes(L->D), L->htab, act_table_bytes(L->dff), L->hpart, nseg,
            nullptr, nullptr, 1};
   hipLaunchKernelGGL((gate_up_eg_kernel<Q4, RG, NTW, D, NW>), dim3(tpad * (unsigned)nseg), dim3(64 * NW),
-                     C::BYTES, s, g);
+                     lds, s, g);
   moe_status st = check_hip(hipGetLastError(), "expert gate/up launch");
   if (st) return st;
   // down: row tiles per block (kDownRowTiles at most; one for a partial
@@ -897,7 +945,7 @@ moe_status launch_eg_shape(const LayerDev* L, int ntask, hipStream_t s) {
   EgArgs d{L->dq, nullptr, L->ds, nullptr, L->rbd, L->D, L->dff, L->topk, L->perm, L->tasks, ntask,
            L->htab, act_table_bytes(L->dff), nullptr, 0, L->hpart, nseg, L->y, L->y16, rtpb};
   hipLaunchKernelGGL((down_eg_kernel<Q4, RG, NTW, D, NW>),
-                     dim3(tpad * (unsigned)((nrt + rtpb - 1) / rtpb)), dim3(64 * NW), C::BYTES, s, d);
+                     dim3(tpad * (unsigned)((nrt + rtpb - 1) / rtpb)), dim3(64 * NW), lds, s, d);
   return check_hip(hipGetLastError(), "expert down launch");
 }
 
