@@ -16,6 +16,8 @@
 // Shapes without a tiled geometry (row bytes not LPR*P*16, unaligned rows,
 // odd-K Q4) and Q4 activations that need 4 limbs use a one-wave-per-row
 // kernel with plain int32 arithmetic on the fp32 activations.
+#include <algorithm>
+#include <climits>
 #include <cstdlib>
 
 #include "moe_device.h"
@@ -284,6 +286,175 @@ __global__ __launch_bounds__(kBlock) void qgemv_fused(TiledArgs a) {
   gemv_write_outputs(ybuf, kYRows, job.C, a.sh.ldc, mbase, ntok, r0, r1);
 }
 
+// Shapes without a tiled geometry: any row bytes from 16 up, any alignment.
+// A row is cut into 16-byte chunks, the last one moved back to end with the
+// row (its activations are zero where it overlaps the chunk before), read
+// with unaligned 16-byte loads, so nothing past a row is read.  Each block
+// quantizes its MT tokens' activations into LDS once (16-byte units per
+// chunk and limb: Q8 the 16 columns, Q4 the 16 even columns, then the 16 odd
+// ones), then L lanes share a row, RPT rows a lane, each unit read from LDS
+// serving RPT rows.  Activations past two limbs take the exact fp32
+// fallback.
+//
+// Bound: latency at a few MB (each block: its activations, two or three
+// dependent chunk loads, the reduction).  Q8 [1000 x 1030], 7 tokens: 20.2
+// us with one wave a row converting every activation per row, 7.9 us here;
+// [4096 x 4000], 64 tokens: 553 -> 37.
+typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(1)));
+
+struct AnyArgs {
+  QShape sh;
+  const QJob* jobs;
+  QJob one;
+  int blocks_per_job;
+  int rows_per_block;
+};
+
+struct AnyEpi {
+  const float* S;
+  float* C;
+  float div;
+  __device__ void operator()(int row, const uint32_t (&tot)[1][1]) const {
+    C[row] = qdot_epilogue(tot[0][0], div, S[row]);
+  }
+};
+
+template <bool Q4, int MT, int L, int RPT>
+__global__ __launch_bounds__(kBlock) void qgemv_any(AnyArgs a) {
+  constexpr int U = Q4 ? 2 : 1;          // 16-byte units per chunk and limb
+  constexpr int G = kWave / L;           // row groups of a wave
+  extern __shared__ u32x4 any_lds[];     // [MT][2 limbs][NC][U]
+  __shared__ int nl_s;
+  __shared__ uint32_t asum[MT];
+  uint8_t* act = reinterpret_cast<uint8_t*>(any_lds);
+  const int K = a.sh.K, rb = Q4 ? K / 2 : K;
+  const int NC = (rb + 15) / 16;
+  const int job_id = blockIdx.x / a.blocks_per_job;
+  const int r0 = (blockIdx.x % a.blocks_per_job) * a.rows_per_block;
+  const int r1 = min(r0 + a.rows_per_block, a.sh.N);
+  const QJob job = a.jobs ? a.jobs[job_id] : a.one;
+  const int m0 = blockIdx.y * MT, ntok = min(MT, a.sh.M - m0);
+  const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
+  const float div = Q4 ? 7.0f : 127.0f;
+  if (tid == 0) nl_s = 1;
+  if (tid < MT) asum[tid] = 0u;
+  // the last chunk's bytes that repeat the chunk before
+  const int dup = 16 * NC - rb;
+  for (int i = tid; i < MT * 2 * U * 16; i += kBlock) {
+    const int u = i / 16, o = i % 16;
+    if (o < dup) act[((size_t)(u / U) * NC * U + (size_t)(NC - 1) * U + u % U) * 16 + o] = 0;
+  }
+  __syncthreads();
+  // quantize: column k of byte position p (Q8 k, Q4 k / 2) sits in chunk
+  // p / 16, the last chunk starting at byte rb - 16
+  int32_t lo = 0, hi = 0;   // limbs_needed is monotone in |value|
+  uint32_t sum[MT];
+#pragma unroll
+  for (int t = 0; t < MT; ++t) sum[t] = 0u;
+  for (int k = tid; k < K; k += kBlock) {
+    float x[MT];
+#pragma unroll
+    for (int t = 0; t < MT; ++t) x[t] = job.A[(size_t)(m0 + min(t, ntok - 1)) * a.sh.lda + k];
+    const int pos = Q4 ? k / 2 : k;
+    const int c = min(pos / 16, NC - 1), o = c < NC - 1 ? pos % 16 : pos - (rb - 16);
+    uint8_t* d = act + ((size_t)c * U + (Q4 ? k % 2 : 0)) * 16 + o;
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+      const int32_t v = f2i_trunc_x86(x[t] * div);
+      lo = min(lo, v);
+      hi = max(hi, v);
+      uint32_t b[4];
+      split_limbs(v, b);
+      d[(size_t)(2 * t) * NC * U * 16] = (uint8_t)b[0];
+      d[(size_t)(2 * t + 1) * NC * U * 16] = (uint8_t)b[1];
+      sum[t] += (uint32_t)v;
+    }
+  }
+  const int nl = max(limbs_needed(lo), limbs_needed(hi));
+  if (nl > 1) atomicMax(&nl_s, nl);
+  if constexpr (Q4) {
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+      const uint32_t v = group_sum_dpp<kWave>(sum[t]);
+      if (lane == 0) atomicAdd(&asum[t], v);
+    }
+  }
+  __syncthreads();
+  const int nlb = nl_s;
+  if (nlb > 2) {
+    const uint8_t* W[1] = {job.W};
+    for (int t = 0; t < ntok; ++t) {
+      AnyEpi epi{job.S, job.C + (size_t)(m0 + t) * a.sh.ldc, div};
+      generic_rows_fp32<Q4, 1>(W, a.sh.rs, K, job.A + (size_t)(m0 + t) * a.sh.lda, r0, r1, epi, wave, kWaves);
+    }
+    return;
+  }
+  auto run = [&](auto nl_tag) {
+    constexpr int NL = decltype(nl_tag)::value;
+    const int sub = lane / L, l = lane % L;
+    for (int rb0 = r0 + (wave * G + sub) * RPT; rb0 - sub * RPT < r1; rb0 += kWaves * G * RPT) {
+      const uint8_t* w[RPT];
+#pragma unroll
+      for (int i = 0; i < RPT; ++i) w[i] = job.W + (size_t)min(rb0 + i, r1 - 1) * (size_t)a.sh.rs;
+      int acc[RPT][MT][NL];
+#pragma unroll
+      for (int i = 0; i < RPT; ++i)
+#pragma unroll
+        for (int t = 0; t < MT; ++t)
+#pragma unroll
+          for (int n = 0; n < NL; ++n) acc[i][t][n] = 0;
+      auto load = [&](int c, u32x4 (&v)[RPT]) {
+        const int at = min(16 * c, rb - 16);
+#pragma unroll
+        for (int i = 0; i < RPT; ++i) v[i] = *reinterpret_cast<const u32x4_any*>(w[i] + at);
+      };
+      u32x4 cur[RPT], nxt[RPT];
+      if (l < NC) load(l, cur);
+      for (int c = l; c < NC; c += L) {
+        if (c + L < NC) load(c + L, nxt);
+#pragma unroll
+        for (int t = 0; t < MT; ++t)
+#pragma unroll
+          for (int n = 0; n < NL; ++n) {
+            const u32x4* q = any_lds + ((size_t)(2 * t + n) * NC + c) * U;
+            const u32x4 x0 = q[0];
+#pragma unroll
+            for (int i = 0; i < RPT; ++i)
+#pragma unroll
+              for (int d = 0; d < 4; ++d)
+                acc[i][t][n] = dot4(Q4 ? cur[i][d] & 0x0F0F0F0Fu : cur[i][d], x0[d], acc[i][t][n]);
+            if constexpr (Q4) {
+              const u32x4 x1 = q[1];
+#pragma unroll
+              for (int i = 0; i < RPT; ++i)
+#pragma unroll
+                for (int d = 0; d < 4; ++d)
+                  acc[i][t][n] = dot4((cur[i][d] >> 4) & 0x0F0F0F0Fu, x1[d], acc[i][t][n]);
+            }
+          }
+#pragma unroll
+        for (int i = 0; i < RPT; ++i) cur[i] = nxt[i];
+      }
+#pragma unroll
+      for (int i = 0; i < RPT; ++i) {
+        const int row = rb0 + i;
+        const float sc = job.S[min(row, r1 - 1)];
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+          uint32_t v = (uint32_t)acc[i][t][0];
+          if constexpr (NL == 2) v += (uint32_t)acc[i][t][1] << 8;
+          v = group_sum_dpp<L>(v);
+          if constexpr (Q4) v -= 8u * asum[t];
+          if (l == 0 && t < ntok && row < r1)
+            job.C[(size_t)(m0 + t) * a.sh.ldc + row] = qdot_epilogue(v, div, sc);
+        }
+      }
+    }
+  };
+  if (nlb == 1) run(std::integral_constant<int, 1>());
+  else run(std::integral_constant<int, 2>());
+}
+
 template <bool Q4>
 __global__ __launch_bounds__(kBlock) void qgemv_generic(QShape sh, const QJob* __restrict__ jobs,
                                                         QJob one, int blocks_per_job) {
@@ -548,6 +719,56 @@ bool qgemv_tiled_ok(const QShape& sh, const void* w_base) {
   return select_tiled(sh, w_base, &v);
 }
 
+// qgemv_any where its tables fit (false: the caller runs qgemv_generic):
+// even Q4 columns, rows of at least one chunk, two limbs of MT tokens within
+// 129 KB of LDS.  MT: 1, 4 or 8 tokens a block.  A whole wave per row while the rows
+// are few (the launch is latency-bound then), 16 lanes per row where a row
+// has under 32 chunks; with several tokens and 4096 rows or more, 16 lanes
+// and four rows each, so that one LDS read serves four rows.
+bool launch_any(const QShape& sh, const QJob* jobs_dev, const QJob& one, int njobs, hipStream_t stream,
+                hipError_t* err) {
+  const bool q4 = sh.dtype == 3;
+  const long long rb = q4 ? sh.K / 2 : sh.K;
+  if ((q4 && (sh.K & 1)) || rb < 16 || sh.K > 65536 || sh.rs != rb) return false;
+  int mt = sh.M == 1 ? 1 : sh.M <= 4 ? 4 : 8;
+  while (mt > 1 && (long long)mt * sh.K > 65536) mt = mt == 8 ? 4 : 1;
+  const int nc = (int)((rb + 15) / 16);
+  const bool wide = mt > 1 && sh.N >= 4096;
+  const int L = wide || nc < 32 ? 16 : 64, rpt = wide ? 4 : 1;
+  const int unit = kWaves * (kWave / L) * rpt;
+  const long long units = ((long long)sh.N + unit - 1) / unit;
+  const long long per = std::max<long long>(1, (units * njobs + 2047) / 2048);   // at most ~2048 blocks a token group
+  AnyArgs a{sh, jobs_dev, one, (int)((units + per - 1) / per), (int)std::min<long long>(per * unit, INT_MAX / 2)};
+  const long long gx = (long long)a.blocks_per_job * njobs, gy = (sh.M + mt - 1) / mt;
+  if (gx > INT_MAX || gy > 65535) return false;
+  *err = hipSuccess;
+  const size_t lds = (size_t)mt * 2 * nc * (q4 ? 2 : 1) * 16;
+  const dim3 grid((unsigned)gx, (unsigned)gy);
+  auto go = [&](auto q4_tag, auto mt_tag, auto l_tag, auto r_tag) {
+    auto* fn = qgemv_any<decltype(q4_tag)::value, decltype(mt_tag)::value, decltype(l_tag)::value,
+                         decltype(r_tag)::value>;
+    if (lds > 60 * 1024)
+      *err = hipFuncSetAttribute((const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (*err != hipSuccess) return;
+    hipLaunchKernelGGL(fn, grid, dim3(kBlock), lds, stream, a);
+    *err = hipGetLastError();
+  };
+  using std::integral_constant;
+  auto with_mt = [&](auto q4_tag, auto mt_tag) {
+    if (wide) go(q4_tag, mt_tag, integral_constant<int, 16>(), integral_constant<int, 4>());
+    else if (L == 16) go(q4_tag, mt_tag, integral_constant<int, 16>(), integral_constant<int, 1>());
+    else go(q4_tag, mt_tag, integral_constant<int, 64>(), integral_constant<int, 1>());
+  };
+  auto with_q = [&](auto q4_tag) {
+    if (mt == 8) with_mt(q4_tag, integral_constant<int, 8>());
+    else if (mt == 4) with_mt(q4_tag, integral_constant<int, 4>());
+    else with_mt(q4_tag, integral_constant<int, 1>());
+  };
+  if (q4) with_q(std::true_type());
+  else with_q(std::false_type());
+  return true;
+}
+
 hipError_t launch_qgemv(const QShape& sh, const QJob* jobs_dev, const QJob& one, int njobs,
                         hipStream_t stream) {
   if (sh.M <= 0 || sh.N <= 0 || njobs <= 0) return hipSuccess;
@@ -569,6 +790,8 @@ hipError_t launch_qgemv(const QShape& sh, const QJob* jobs_dev, const QJob& one,
     if (e != hipSuccess) return e;
     return launch_qgemv_tables(sh, jobs_dev, one, njobs, g_ws, 0, stream);
   }
+  hipError_t err;
+  if (launch_any(sh, jobs_dev, one, njobs, stream, &err)) return err;
   const int bpj = (sh.N + kWaves - 1) / kWaves;
   dim3 grid((unsigned)((long long)bpj * njobs), (unsigned)((sh.M + 15) / 16));
   if (sh.dtype == 3)

@@ -1,0 +1,47 @@
+"""The untiled-shape GEMV kernel (unaligned 16-byte row chunks, activations
+quantized per block) against the oracle, bit for bit."""
+import numpy as np
+import pytest
+
+import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def bits(a):
+    return np.ascontiguousarray(a, dtype=np.float32).view(np.uint32)
+
+
+# (dtype, N, K): rows of exactly one chunk, one byte more, whole chunks, a
+# last chunk that repeats 15 bytes; 31 / 32 / 33 chunks (16 lanes a row below
+# 32, a wave from 32), 64 and 65 chunks (one and two per lane); 4096 rows and
+# more with several tokens (four rows a lane); the largest K of each token
+# count (8 x 8192, 4 x 16384, 1 x 65536) and one past
+SHAPES = [(2, 5, 16), (2, 7, 17), (2, 9, 48), (2, 33, 31), (2, 20, 496), (2, 20, 511), (2, 17, 513),
+          (2, 130, 1023), (2, 130, 1030), (2, 4099, 66), (2, 9, 8191), (2, 9, 8193), (2, 6, 16385),
+          (2, 3, 65535), (2, 3, 65537),
+          (3, 5, 32), (3, 7, 34), (3, 33, 62), (3, 20, 992), (3, 17, 1026), (3, 130, 2050),
+          (3, 4097, 70), (3, 9, 8190), (3, 9, 8194), (3, 6, 16386), (3, 3, 65534)]
+
+
+@pytest.mark.parametrize("dtype,N,K", SHAPES)
+@pytest.mark.parametrize("M,scale", [(1, 1.0), (4, 0.05), (5, 30.0), (9, 1.0), (2, 1e5)])
+def test_gemv_any_shapes(moehip, dtype, N, K, M, scale):
+    print("gemv any case", dtype, N, K, M, scale, flush=True)
+    assert moehip.gemv_variant(dtype, M, N, K) == "generic"
+    seed = dtype * 100000 + N * 31 + K * 7 + M
+    A = O.normal(M * K, seed, 0.0, scale).reshape(M, K)
+    rb = K if dtype == 2 else K // 2
+    q = (O.uniform_u32(N * rb, seed + 1) & 0xFF).astype(np.uint8)
+    q = (q.view(np.int8) if dtype == 2 else q).reshape(N, rb)
+    s = O.normal(N, seed + 2, 0.0, 0.01)
+    want = (O.gemv_q8 if dtype == 2 else O.gemv_q4)(A, q, s, N, K)
+    L = moehip.lib()
+    # the weights from an odd address, with bytes of another value around them
+    raw = np.full(rb * N + 65, 0x5A, np.uint8)
+    raw[33:33 + rb * N] = q.reshape(-1).view(np.uint8)
+    dA, dq, ds = (moehip.DeviceBuffer.from_array(v) for v in (A, raw, s))
+    dC = moehip.DeviceBuffer(M * N * 4)
+    f = L.moe_matmul_q8_dev if dtype == 2 else L.moe_matmul_q4_dev
+    moehip.check(f(dA.ptr, dq.ptr + 33, ds.ptr, dC.ptr, M, N, K), "gemv")
+    np.testing.assert_array_equal(bits(dC.download((M, N), np.float32)), bits(want))
