@@ -426,9 +426,9 @@ __device__ __forceinline__ v16u fold_limbs(const v16i (&acc)[NTW], int t, int l)
 // Dots of pairs pbase .. over all limbs: one pass for up to LP limbs, else
 // one per LP limbs.  Two limbs a pass read the weights once for both (a pass
 // per limb streamed them from HBM again: gate/up of 300 tokens, Q8, 2-limb
-// activations, 137 -> 87 us; down 75 -> 52).  segmask (down: [3][kEgPairs] in LDS, else
-// null): bit s of segmask[l - 1][pair] says segment s of the pair's h table
-// holds limb plane l.
+// activations, 137 -> 87 us; down 75 -> 52).  segmask (down: [3][kEgPairs] in
+// LDS, else null): bit s of segmask[l - 1][pair] says segment s of the pair's
+// h table holds limb plane l.
 template <bool Q4, int RG, int NTW, int D, int NW, int LP, class WRow>
 __device__ __forceinline__ void eg_dots(WRow&& wrow, int K, const EgPairs& sp, int pbase, int n,
                                         int nl, const uint32_t* segmask, uint8_t* lds,
@@ -970,7 +970,12 @@ bool expert_gemm_ok(const LayerDev* L) {
 
 int expert_gemm_tiles(const LayerDev* L, int T) {
   const int mean = T * L->topk / (L->E > 0 ? L->E : 1);
-  return mean <= 24 ? 1 : (mean <= 64 ? 2 : 4);
+  // Layer times at 128 experts, top-8 (us), 32- / 64- / 256-pair shape: Q8 T =
+  // 300 (mean 18) 171 / 188 / 193, 512 (32) 222 / 207 / 213, 700 (43) 256 / 227
+  // / 234, 1024 (64: half the experts' pairs split over two 64-pair tasks) 313
+  // / 306 / 261; Q4 300 114 / 125 / 128, 512 142 / 133 / 142, 700 166 / 148 /
+  // 155, 1024 196 / 188 / 173.
+  return mean <= 24 ? 1 : (mean <= 48 ? 2 : 4);
 }
 
 int expert_gemm_split(int nt) { return nt == 4 ? 256 : 32 * nt; }
