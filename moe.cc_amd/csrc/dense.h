@@ -94,12 +94,13 @@ moe_status heads_norm_rope(const HeadArgs& a, hipStream_t s);
 
 // Causal attention of the T new rows (test_model_trace.c:404-426): scores
 // S[t][h][tk] = (q . k_tk) * scale for tk <= pos0 + t, then the softmax and
-// the weighted V sum into H [T][nq*hd].  S is scratch [T][nq][max_seq].
+// the weighted V sum into H [T][nq*hd].  S is scratch [T][nq][ss], ss >=
+// max_seq (a multiple of 4 for the many-row kernels' 16-byte loads).
 struct AttnArgs {
   const float* qkv; int ld;
   float* kc; float* vc;
   float* S; float* H;
-  int T, pos0, nq, nkv, hd, max_seq;
+  int T, pos0, nq, nkv, hd, max_seq, ss;
   float scale;
   // T == 1 only: the score launch also does heads_norm_rope's work for its
   // row (q/k norm, RoPE, K and V into the caches); qkv holds the raw

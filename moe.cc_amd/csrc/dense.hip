@@ -635,6 +635,15 @@ __global__ __launch_bounds__(kRowFinishWaves * kWave) void row_finish_kernel(Den
 // product floor of the first is 148.
 typedef float v16f __attribute__((ext_vector_type(16)));
 
+// The products of 16 columns of a 16 x 16 tile (x, w: the lane's columns 4b ..
+// 4b + 3 of its token and row): p[c][4b + r] belongs to column 4b + c, chain r.
+__device__ __forceinline__ void mfma_products(const float4& x, const float4& w, v16f (&p)[4]) {
+  p[0] = __builtin_amdgcn_mfma_f32_16x16x1f32(x.x, w.x, v16f{}, 0, 0, 0);
+  p[1] = __builtin_amdgcn_mfma_f32_16x16x1f32(x.y, w.y, v16f{}, 0, 0, 0);
+  p[2] = __builtin_amdgcn_mfma_f32_16x16x1f32(x.z, w.z, v16f{}, 0, 0, 0);
+  p[3] = __builtin_amdgcn_mfma_f32_16x16x1f32(x.w, w.w, v16f{}, 0, 0, 0);
+}
+
 __device__ __align__(16) const float kDenseZero[4] = {};
 
 template <int WX, int NB, int KC, int D>
@@ -701,10 +710,7 @@ __global__ __launch_bounds__(256, 4) void dense_mfma_kernel(DenseArgs a) {
       }
       asm volatile("" ::: "memory");   // the next step's operands are requested here, not sunk to their use
       v16f p[4];
-      p[0] = __builtin_amdgcn_mfma_f32_16x16x1f32(x.x, w.x, v16f{}, 0, 0, 0);
-      p[1] = __builtin_amdgcn_mfma_f32_16x16x1f32(x.y, w.y, v16f{}, 0, 0, 0);
-      p[2] = __builtin_amdgcn_mfma_f32_16x16x1f32(x.z, w.z, v16f{}, 0, 0, 0);
-      p[3] = __builtin_amdgcn_mfma_f32_16x16x1f32(x.w, w.w, v16f{}, 0, 0, 0);
+      mfma_products(x, w, p);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int k = 0; k < 16; ++k)
@@ -799,41 +805,75 @@ __device__ void heads_prep(float* v0, float* v1, const float* w0, const float* w
   }
 }
 
-// Block (t, h) over the heads of row t of [Q | K | V] (each head hd wide, so
-// head h starts at h * hd): q/k heads through heads_prep at position
-// pos0 + t (Q stays in place, K goes to the cache), V rows to the cache.
-__global__ __launch_bounds__(64) void heads_kernel(HeadArgs a) {
-  __shared__ float4 v4[kMaxHd / 4];
-  __shared__ float4 sq4[2 * kMaxHd / 4];
-  __shared__ float4 w4[kMaxHd / 4];
-  __shared__ float4 cs4[kMaxHd / 8], sn4[kMaxHd / 8];
-  __shared__ float inv_s[2];
-  const int t = blockIdx.x, h = blockIdx.y, lane = threadIdx.x;
-  const int hd = a.hd, d2 = hd / 2, pos = a.pos0 + t;
-  float* row = a.qkv + (size_t)t * a.ld + (size_t)h * hd;
-  if (h >= a.nq + a.nkv) {   // V head: into the cache unchanged
-    float* dst = a.vc + ((size_t)(h - a.nq - a.nkv) * a.max_seq + pos) * hd;
-    for (int d = lane; d < hd; d += 64) dst[d] = row[d];
-    return;
+// kHeadRows consecutive (token, head) rows of [Q | K | V] a block (row q is
+// head q % (nq + 2 nkv) of token q / (nq + 2 nkv), hd wide): q/k rows through
+// the per-head RMSNorm and RoPE of heads_prep at position pos0 + t (Q in
+// place, K to the cache), V rows to the cache unchanged.  One lane a row runs
+// its sequential sum of squares, 16 rows side by side (one row a block left
+// the chip waiting on 20,480 such chains: 512 tokens, 40 heads of 128, 18.6 ->
+// 8.9 us).
+constexpr int kHeadRows = 16;
+
+__global__ __launch_bounds__(256) void heads_kernel(HeadArgs a) {
+  extern __shared__ float hrow[];   // [kHeadRows][hd + 4] rows, then the same of squares
+  __shared__ float inv_s[kHeadRows];
+  constexpr int RW = kHeadRows / 4;   // rows a wave
+  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+  const int hd = a.hd, d2 = hd / 2, LD = hd + 4, H = a.nq + 2 * a.nkv;
+  const long long q0 = (long long)blockIdx.x * kHeadRows, nrow = (long long)a.T * H;
+  float* sq = hrow + kHeadRows * LD;
+  float* row[RW];
+  int t[RW], h[RW];
+#pragma unroll
+  for (int i = 0; i < RW; ++i) {
+    const long long q = min(q0 + wave * RW + i, nrow - 1);
+    t[i] = (int)(q / H);
+    h[i] = (int)(q % H);
+    row[i] = a.qkv + (size_t)t[i] * a.ld + (size_t)h[i] * hd;
   }
-  const bool isq = h < a.nq;
-  const float* wg = isq ? a.q_norm : a.k_norm;
-  float* v = reinterpret_cast<float*>(v4);
-  float* w = reinterpret_cast<float*>(w4);
-  float* cs = reinterpret_cast<float*>(cs4);
-  float* sn = reinterpret_cast<float*>(sn4);
-  for (int d = lane; d < hd; d += 64) {
-    v[d] = row[d];
-    if (wg) w[d] = wg[d];
-  }
-  for (int i = lane; i < d2; i += 64) {
-    cs[i] = a.rope_cos[(size_t)pos * d2 + i];
-    sn[i] = a.rope_sin[(size_t)pos * d2 + i];
+  for (int d = lane; d < hd; d += kWave) {
+    float v[RW];
+#pragma unroll
+    for (int i = 0; i < RW; ++i) v[i] = row[i][d];
+#pragma unroll
+    for (int i = 0; i < RW; ++i) {
+      hrow[(wave * RW + i) * LD + d] = v[i];
+      sq[(wave * RW + i) * LD + d] = v[i] * v[i];
+    }
   }
   __syncthreads();
-  float* out = isq ? row : a.kc + ((size_t)(h - a.nq) * a.max_seq + pos) * hd;
-  heads_prep(v, nullptr, wg ? w : nullptr, nullptr, a.eps, hd, cs, sn, reinterpret_cast<float*>(sq4),
-             inv_s, out, nullptr);
+  if ((int)threadIdx.x < kHeadRows) {
+    const float msq = chain_sum(0.0f, sq + threadIdx.x * LD, hd / 4);
+    inv_s[threadIdx.x] = 1.0f / sqrtf(msq / (float)hd + a.eps);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < RW; ++i) {
+    if (q0 + wave * RW + i >= nrow) break;
+    const int pos = a.pos0 + t[i];
+    const float* v = hrow + (wave * RW + i) * LD;
+    if (h[i] >= a.nq + a.nkv) {
+      float* dst = a.vc + ((size_t)(h[i] - a.nq - a.nkv) * a.max_seq + pos) * hd;
+      for (int d = lane; d < hd; d += kWave) dst[d] = v[d];
+      continue;
+    }
+    const float* w = h[i] < a.nq ? a.q_norm : a.k_norm;
+    float* out = h[i] < a.nq ? row[i] : a.kc + ((size_t)(h[i] - a.nq) * a.max_seq + pos) * hd;
+    const float inv = inv_s[wave * RW + i];
+    for (int d = lane; d < d2; d += kWave) {
+      float e = v[d], o = v[d + d2];
+      if (w) {
+        e = e * inv;
+        o = o * inv;
+        e = e * w[d];
+        o = o * w[d + d2];
+      }
+      const float c = a.rope_cos[(size_t)pos * d2 + d], s = a.rope_sin[(size_t)pos * d2 + d];
+      const float ec = e * c, os = o * s, oc = o * c, es = e * s;
+      out[d] = ec - os;
+      out[d + d2] = oc + es;
+    }
+  }
 }
 
 // ---------------------------------------------------------------- attention
@@ -1174,209 +1214,291 @@ __global__ __launch_bounds__(kPvThreads) void attn_softmax_pv_kernel(AttnArgs a)
   }
 }
 
-// ---- many query rows (prefill): several rows share each staged K / V tile ----
+// ---- many query rows (prefill) ----
 //
-// The one-row kernels above read the whole key / value prefix once per
-// query row (T^2/2 rows of hd floats for T new rows); these read it once per
-// kSq (scores) or kQt (softmax and V sums) rows.  Same chains, same order:
-// bit-identical results.
-constexpr int kQt = 8;
+// The one-row kernels above read the whole key / value prefix once per query
+// row; these read it once per 32 rows, with the products on the matrix cores
+// and the chains' adds on the VALU as in dense_mfma_kernel (its operand
+// layout: lane (b, j) = (lane / 16, lane % 16), MFMA c of 16 columns has
+// column 4b + c in block b, result register 4b' + r of MFMA c the product of
+// chain r and column 4b' + c).  Same chains, same order: bit-identical
+// results.  512 rows, 32 / 4 heads of 128: scores 71 -> 32 us, V sums 74 -> 26
+// (15 of each are the products and adds at 4.3 clocks per 64), softmax 18.
 
-// Scores of query rows t0 .. t0 + kSq - 1 (t0 = kSq blockIdx.z) of head
-// blockIdx.y against keys tk0 .. tk0 + 63 (tk0 = 64 blockIdx.x): K rows and
-// queries staged in LDS with coalesced loads; wave w runs the chains of rows
-// w, w + 4, w + 8, w + 12 side by side, lane = key.  q must already be
-// normed and rotated (heads_kernel).  S as attn_scores_kernel, key <= pos0 +
-// t only.
-constexpr int kSq = 16;                 // query rows per block
-constexpr int kSqPerWave = kSq / 4;     // chains per lane
+// The head of block x of a grid whose x runs over the nq heads: blocks are
+// dealt to the 8 XCDs in turn, so XCD k takes heads k nq/8 .. and a KV head's
+// rows come from few XCDs' L2s.  Heads run fastest in these grids: with the key
+// chunks fastest, XCD 0 took the keys that every row sees (43 us of scores
+// against 34).
+__device__ __forceinline__ int attn_head(int x, int nq) {
+  return nq % 8 ? x : x % 8 * (nq / 8) + x / 8;
+}
 
-__global__ __launch_bounds__(256) void attn_scores_qt_kernel(AttnArgs a) {
-  extern __shared__ float lds[];
-  const int hd = a.hd, h4 = hd / 4, LD = hd + 4;
-  float* kt = lds;             // [64][LD]
-  float* qs = kt + 64 * LD;    // [kSq][hd]
-  const int h = blockIdx.y, t0 = blockIdx.z * kSq, tk0 = blockIdx.x * 64;
-  const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
-  const int nt = min(kSq, a.T - t0);
-  const int Pmax = a.pos0 + t0 + nt - 1;
+// Scores of query rows t0 .. t0 + 31 of one head against
+// kSkt tiles of 32 keys from 128 blockIdx.y on; wave w: rows 16 (w %
+// 2) .., keys 16 (w / 2) .. of each tile.  The queries stay in LDS, the key
+// tiles stream through a ring of D buffers in stages of 64 columns (nh stages
+// a tile, columns past hd zero), so that only a block's first loads are waited
+// for (one tile a block: 45 us at 512 rows, most of it blocks waiting for
+// their own two loads).  q must already be normed and rotated (heads_kernel).
+// S rows (head, token) are a.ss apart; key <= pos0 + t only is written.
+constexpr int kSq = 32, kSk = 32, kSkt = 4;
+constexpr int kSkD = 3;
+constexpr int kStageB = 32 * 64 * 4;   // bytes of 32 rows x 64 columns
+
+__global__ __launch_bounds__(256, 4) void attn_scores_qt_kernel(AttnArgs a) {
+  constexpr int SL = 16, NL = 2;   // 16-byte slots of a row; load instructions of a stage per wave
+  extern __shared__ float4 sq4[];  // [nh] query stages, [kSkD] key stages
+  const int hd = a.hd, nh = (hd + 63) / 64;
+  const int h = attn_head(blockIdx.x, a.nq), tk0 = blockIdx.y * (kSk * kSkt);
+  const int t0 = ((int)gridDim.z - 1 - (int)blockIdx.z) * kSq;
+  const int Pmax = min(a.pos0 + t0 + kSq, a.pos0 + a.T) - 1;
   if (tk0 > Pmax) return;   // every key of the block is masked (uniform)
+  const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int b = lane / 16, j = lane % 16, wx = wave % 2, wn = wave / 2;
   const int kvh = h / (a.nq / a.nkv);
-  const int rows = min(64, Pmax + 1 - tk0);
-  const float* kbase = a.kc + ((size_t)kvh * a.max_seq + tk0) * hd;
-  // K rows (rows past `rows` read row rows - 1; never used), then the queries
-  // (rows past nt read row nt - 1)
-  for (int base = 0; base < 64 * h4; base += 256 * 8) {
-    float4 r[8];
+  const float* kbase = a.kc + (size_t)kvh * a.max_seq * hd;
+  const int steps = min(kSkt, (Pmax - tk0) / kSk + 1) * nh;
+  uint8_t* qlds = reinterpret_cast<uint8_t*>(sq4);
+  uint8_t* klds = qlds + nh * kStageB;
+  // instruction v of a stage: rows 4 (wave + 4v) + lane / 16
+  int row[NL], col[NL];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int i = base + tid + 256 * u, rr = min(i / h4, rows - 1);
-      r[u] = i < 64 * h4 ? *reinterpret_cast<const float4*>(kbase + (size_t)rr * hd + 4 * (i % h4)) : zero4();
+  for (int v = 0; v < NL; ++v) {
+    row[v] = 4 * (wave + 4 * v) + lane / SL;
+    col[v] = 4 * ((lane % SL) ^ (row[v] & 15));
+  }
+  auto load_k = [&](int s, int buf) {
+    const int key0 = tk0 + kSk * (s / nh), c0 = 64 * (s % nh);
+#pragma unroll
+    for (int v = 0; v < NL; ++v)
+      lds_load16(c0 + col[v] < hd ? kbase + (size_t)min(key0 + row[v], Pmax) * hd + c0 + col[v] : kDenseZero,
+                 klds + buf * kStageB + (wave + 4 * v) * 1024);
+  };
+  for (int c = 0; c < nh; ++c)
+#pragma unroll
+    for (int v = 0; v < NL; ++v)
+      lds_load16(64 * c + col[v] < hd
+                     ? a.qkv + (size_t)min(t0 + row[v], a.T - 1) * a.ld + (size_t)h * hd + 64 * c + col[v]
+                     : kDenseZero,
+                 qlds + c * kStageB + (wave + 4 * v) * 1024);
+#pragma unroll
+  for (int p = 0; p < kSkD - 1; ++p) load_k(min(p, steps - 1), p);
+  float acc[4] = {}, done[4];
+  auto put = [&](int tile) {   // the finished tile's scores
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int tok = t0 + 16 * wx + 4 * b + r, key = tk0 + kSk * tile + 16 * wn + j;
+      if (tok < a.T && key <= a.pos0 + tok) a.S[((size_t)h * a.T + tok) * a.ss + key] = done[r] * a.scale;
     }
+  };
+  for (int s = 0; s < steps; ++s) {
+    stage_sync<(kSkD - 2) * NL>();
+    // a tile's stores go out before the next loads, so that the wait above
+    // counts them only a whole stage later
+    if (s && s % nh == 0) put(s / nh - 1);
+    load_k(min(s + kSkD - 1, steps - 1), (s + kSkD - 1) % kSkD);
+    const float4* Q = reinterpret_cast<const float4*>(qlds + (s % nh) * kStageB) + (16 * wx + j) * SL;
+    const float4* B = reinterpret_cast<const float4*>(klds + (s % kSkD) * kStageB) + (16 * wn + j) * SL;
+    float4 x = Q[b ^ j], w = B[b ^ j];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int i = base + tid + 256 * u;
-      if (i < 64 * h4) *reinterpret_cast<float4*>(kt + (i / h4) * LD + 4 * (i % h4)) = r[u];
+    for (int g = 0; g < 4; ++g) {
+      float4 xn = x, wn4 = w;
+      if (g + 1 < 4) {
+        xn = Q[(4 * (g + 1) + b) ^ j];
+        wn4 = B[(4 * (g + 1) + b) ^ j];
+      }
+      asm volatile("" ::: "memory");
+      v16f p[4];
+      mfma_products(x, w, p);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int k = 0; k < 16; ++k)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[r] = acc[r] + p[k % 4][4 * (k / 4) + r];
+      __builtin_amdgcn_sched_barrier(0);
+      x = xn;
+      w = wn4;
     }
-  }
-  for (int i = tid; i < kSq * h4; i += 256) {
-    const int qr = min(i / h4, nt - 1);
-    *reinterpret_cast<float4*>(qs + (i / h4) * hd + 4 * (i % h4)) =
-        *reinterpret_cast<const float4*>(a.qkv + (size_t)(t0 + qr) * a.ld + (size_t)h * hd + 4 * (i % h4));
-  }
-  __syncthreads();
-  const int key = tk0 + lane;
-  if (lane >= rows) return;
-  const float4* k4 = reinterpret_cast<const float4*>(kt + lane * LD);
-  float dot[kSqPerWave];
+    if (s % nh == nh - 1) {
 #pragma unroll
-  for (int u = 0; u < kSqPerWave; ++u) dot[u] = 0.0f;
-  for (int c = 0; c < h4; ++c) {
-    const float4 k = k4[c];
-    float4 x[kSqPerWave];
-#pragma unroll
-    for (int u = 0; u < kSqPerWave; ++u) x[u] = reinterpret_cast<const float4*>(qs + (wave + 4 * u) * hd)[c];
-    float p[kSqPerWave][4];
-#pragma unroll
-    for (int u = 0; u < kSqPerWave; ++u) {
-      p[u][0] = x[u].x * k.x;
-      p[u][1] = x[u].y * k.y;
-      p[u][2] = x[u].z * k.z;
-      p[u][3] = x[u].w * k.w;
-    }
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-#pragma unroll
-      for (int u = 0; u < kSqPerWave; ++u) dot[u] = dot[u] + p[u][e];
-  }
-#pragma unroll
-  for (int u = 0; u < kSqPerWave; ++u) {
-    const int q = wave + 4 * u;
-    if (q < nt && key <= a.pos0 + t0 + q) a.S[((size_t)(t0 + q) * a.nq + h) * a.max_seq + key] = dot[u] * a.scale;
-  }
-}
-
-// Softmax of the score rows of the query-tiled path, in place, once per
-// (query row, head): one wave each, row t of head h (n = pos0 + t + 1
-// scores) staged in LDS; its max by the wave (order-free; a NaN first score
-// wins, as in attn_softmax_pv_kernel), e = expf(s - m), the sum chain in
-// lane 0, p = e * (1 / (sum + 1e-9)) written back over the scores
-// (test_model_trace.c:411-420).  attn_pv_qt_kernel then reads p.
-constexpr int kSmRowWaves = 4;
-
-size_t attn_softmax_rows_lds(int pos0, int T) {
-  return (size_t)kSmRowWaves * (size_t)((pos0 + T + 3) & ~3) * 4;
-}
-
-__global__ __launch_bounds__(kSmRowWaves * kWave) void attn_softmax_rows_kernel(AttnArgs a) {
-  extern __shared__ float smr[];   // [kSmRowWaves][ES]
-  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-  const int h = blockIdx.x * kSmRowWaves + wave, t = blockIdx.y;
-  if (h >= a.nq) return;   // (no block barriers below)
-  const int ES = (a.pos0 + a.T + 3) & ~3;
-  float* er = smr + (size_t)wave * ES;
-  const int n = a.pos0 + t + 1;
-  float* Srow = a.S + ((size_t)t * a.nq + h) * a.max_seq;
-  float mx = -__builtin_inff();
-  for (int i = lane; i < n; i += kWave) {
-    const float v = Srow[i];
-    er[i] = v;
-    if (v == v && v > mx) mx = v;
-  }
-#pragma unroll
-  for (int off = kWave / 2; off > 0; off >>= 1) {
-    const float o = __shfl_xor(mx, off, kWave);
-    mx = o > mx ? o : mx;
-  }
-  __threadfence_block();
-  __builtin_amdgcn_wave_barrier();
-  const float s0 = er[0];
-  const float m = s0 != s0 ? s0 : mx;
-  for (int i = lane; i < n; i += kWave) er[i] = expf_glibc(er[i] - m);
-  for (int i = n + lane; i < ((n + 3) & ~3); i += kWave) er[i] = 0.0f;
-  __threadfence_block();
-  __builtin_amdgcn_wave_barrier();
-  float inv = 0.0f;
-  if (lane == 0) inv = 1.0f / (chain_sum(0.0f, er, (n + 3) / 4) + 1e-9f);
-  inv = __shfl(inv, 0, kWave);
-  for (int i = lane; i < n; i += kWave) Srow[i] = er[i] * inv;
-}
-
-// Weighted V sum of query rows t0 .. t0 + kQt - 1 of head blockIdx.y for
-// dimensions d0 .. d0 + kPvDpb - 1: thread (qi, dd) = (tid / kPvDpb, tid %
-// kPvDpb).  Row qi's probabilities (n = pos0 + t0 + qi + 1, from
-// attn_softmax_rows_kernel) in LDS; V staged kPvCh positions at a time and
-// out = (((0 + p_0 v_0) + p_1 v_1) + ...) over the row's positions in order.
-constexpr int kPvDpb = 32;
-constexpr int kPvCh = 128;
-static_assert(kQt * kPvDpb == 256, "one thread per (row, dimension)");
-
-size_t attn_pv_qt_lds(int pos0, int T) {
-  const size_t es = (size_t)((pos0 + T + 3) & ~3);
-  return ((size_t)kQt * es + (size_t)kPvCh * kPvDpb) * 4;
-}
-
-__global__ __launch_bounds__(256) void attn_pv_qt_kernel(AttnArgs a) {
-  extern __shared__ float lds[];
-  const int hd = a.hd;
-  const int h = blockIdx.y, t0 = blockIdx.z * kQt, d0 = blockIdx.x * kPvDpb;
-  const int tid = threadIdx.x, qi = tid / kPvDpb, dd = tid % kPvDpb;
-  const int ES = (a.pos0 + a.T + 3) & ~3;            // row stride of es
-  float* es = lds;                                    // [kQt][ES]
-  float* vt = es + (size_t)kQt * ES;                  // [kPvCh][kPvDpb]
-  const int nt = min(kQt, a.T - t0);
-  const int nmax = a.pos0 + t0 + nt;                  // positions of the last row
-  const bool row_live = qi < nt;
-  const int n = row_live ? a.pos0 + t0 + qi + 1 : 0;
-  const int kvh = h / (a.nq / a.nkv);
-  float* er = es + (size_t)qi * ES;
-  // 1. the row's probabilities (attn_softmax_rows_kernel)
-  const float* Srow = a.S + ((size_t)(t0 + qi) * a.nq + h) * a.max_seq;
-  for (int i = dd; i < n; i += kPvDpb) er[i] = Srow[i];
-  for (int i = n + dd; i < ((n + 3) & ~3); i += kPvDpb) er[i] = 0.0f;
-  // 2. the weighted V sums
-  const float* vbase = a.vc + (size_t)kvh * a.max_seq * hd + d0;
-  const int dl = min(kPvDpb, hd - d0);
-  float out = 0.0f;
-  for (int c0 = 0; c0 < nmax; c0 += kPvCh) {
-    __syncthreads();   // the previous chunk's readers are done (and p is complete)
-    constexpr int PER = kPvCh * kPvDpb / 4 / 256;   // float4 per thread
-    float4 r[PER];
-#pragma unroll
-    for (int u = 0; u < PER; ++u) {
-      const int i = tid + 256 * u;                  // float4 index in the tile
-      const int pos = c0 + i / (kPvDpb / 4), c = 4 * (i % (kPvDpb / 4));
-      r[u] = (pos < nmax && c < dl) ? *reinterpret_cast<const float4*>(vbase + (size_t)pos * hd + c) : zero4();
-    }
-#pragma unroll
-    for (int u = 0; u < PER; ++u) reinterpret_cast<float4*>(vt)[tid + 256 * u] = r[u];
-    __syncthreads();
-    const int np = min(kPvCh, n - c0);
-    int j = 0;
-    // 16 positions' operands read ahead of their chain steps
-    for (; j + 16 <= np; j += 16) {
-      float4 pe[4];
-      float vv[16];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) pe[u] = *reinterpret_cast<const float4*>(er + c0 + j + 4 * u);
-#pragma unroll
-      for (int u = 0; u < 16; ++u) vv[u] = vt[(j + u) * kPvDpb + dd];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const float p0 = pe[u].x * vv[4 * u], p1 = pe[u].y * vv[4 * u + 1];
-        const float p2 = pe[u].z * vv[4 * u + 2], p3 = pe[u].w * vv[4 * u + 3];
-        out = out + p0;
-        out = out + p1;
-        out = out + p2;
-        out = out + p3;
+      for (int r = 0; r < 4; ++r) {
+        done[r] = acc[r];
+        acc[r] = 0.0f;
       }
     }
-    for (; j < np; ++j) {
-      const float pv = er[c0 + j] * vt[j * kPvDpb + dd];
-      out = out + pv;
+  }
+  put((steps - 1) / nh);
+  stage_sync<0>();   // the clamped loads past the last stage have landed
+}
+
+// Softmax of the score rows, in place (test_model_trace.c:411-420): a block
+// takes R query rows of a head, n = pos0 + t + 1 scores each, staged in LDS
+// (the longest rows' blocks first, those of one length spread over the CUs); max per row by one wave (order-free; a NaN first score wins, as in
+// attn_softmax_pv_kernel), e = expf(s - m), then lane i of wave 0 runs row
+// i's sum chain -- R chains a wave instead of one -- and p = e * (1 / (sum +
+// 1e-9)) goes back over the scores.
+constexpr int kSmRowsMax = 16;
+
+// Floats of a staged row: whole 256-float load instructions, and four so that
+// the 16 lanes of a chain read meet different banks.
+__host__ __device__ constexpr int sm_row_floats(int npos) { return (npos + 255) / 256 * 256 + 4; }
+
+__global__ __launch_bounds__(256) void attn_softmax_rows_kernel(AttnArgs a, int R) {
+  extern __shared__ float smr[];   // [R][LD]
+  __shared__ float inv_s[kSmRowsMax];
+  __shared__ uint64_t exp_tab[32];
+  if (threadIdx.x < 32) exp_tab[threadIdx.x] = kExp2Tab[threadIdx.x];
+  const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int LD = sm_row_floats(a.pos0 + a.T);
+  const int h = attn_head(blockIdx.x, a.nq), t0 = ((int)gridDim.y - 1 - (int)blockIdx.y) * R;
+  const int nr = min(R, a.T - t0);
+  float* S0 = a.S + ((size_t)h * a.T + t0) * a.ss;
+  for (int i = wave; i < nr; i += 4) {
+    const int n = a.pos0 + t0 + i + 1;
+    const float* Srow = S0 + (size_t)i * a.ss;
+    for (int c = 0; c < n; c += 256)
+      lds_load16(c + 4 * lane < a.ss ? Srow + c + 4 * lane : kDenseZero,
+                 reinterpret_cast<uint8_t*>(smr + (size_t)i * LD + c));
+  }
+  stage_sync<0>();
+  for (int i = wave; i < nr; i += 4) {
+    const int n = a.pos0 + t0 + i + 1;
+    float* er = smr + (size_t)i * LD;
+    const float s0 = er[0];
+    float mx = -__builtin_inff();
+    for (int k = lane; k < n; k += kWave) {
+      const float v = er[k];
+      if (v == v && v > mx) mx = v;
+    }
+#pragma unroll
+    for (int off = kWave / 2; off > 0; off >>= 1) {
+      const float o = __shfl_xor(mx, off, kWave);
+      mx = o > mx ? o : mx;
+    }
+    const float m = s0 != s0 ? s0 : mx;
+    // four exponentials side by side (LDS reads, table lookups and fp64 chains)
+    int k = lane;
+    for (; k + 3 * kWave < n; k += 4 * kWave) {
+      float e[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) e[u] = er[k + u * kWave] - m;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) e[u] = expf_glibc_t(e[u], exp_tab);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) er[k + u * kWave] = e[u];
+    }
+    for (; k < n; k += kWave) er[k] = expf_glibc_t(er[k] - m, exp_tab);
+    if (lane < 3 && n + lane < ((n + 3) & ~3)) er[n + lane] = 0.0f;
+  }
+  __syncthreads();
+  if ((int)threadIdx.x < nr) {
+    const int n = a.pos0 + t0 + (int)threadIdx.x + 1;
+    inv_s[threadIdx.x] = 1.0f / (chain_sum(0.0f, smr + (size_t)threadIdx.x * LD, (n + 3) / 4) + 1e-9f);
+  }
+  __syncthreads();
+  for (int i = wave; i < nr; i += 4) {
+    const int n = a.pos0 + t0 + i + 1;
+    float* Srow = S0 + (size_t)i * a.ss;
+    const float* er = smr + (size_t)i * LD;
+    const float inv = inv_s[i];
+    for (int k = lane; k < n; k += kWave) Srow[k] = er[k] * inv;
+  }
+}
+
+// Weighted V sums of query rows t0 .. t0 + 31 of one head for dimensions 64
+// blockIdx.y ..; wave w: rows 16 (w % 2) .., dimensions 32 (w /
+// 2) ...  out = (((0 + p_0 v_0) + p_1 v_1) + ...) over a row's n = pos0 + t + 1
+// positions: chunks of kPvCh positions of p (rows a.ss apart) and V stream
+// through two LDS buffers; a product past the row's n counts as +0, which
+// leaves its chain unchanged (a chain from +0 is never -0).  The longest
+// rows' blocks come first in the grid.
+constexpr int kPvCh = 32;
+
+__global__ __launch_bounds__(256, 3) void attn_pv_qt_kernel(AttnArgs a) {
+  constexpr int PS = kPvCh / 4, VS = 16;                  // 16-byte slots of a p row, a V row (64 dimensions)
+  constexpr int NP = kSq * PS / 64, NV = kPvCh * VS / 64; // load instructions
+  static_assert(NP == 4 && NV == 8, "whole instructions per wave");
+  __shared__ float4 lds4[2][kSq * PS + kPvCh * VS];
+  const int hd = a.hd, h = attn_head(blockIdx.x, a.nq), d0 = blockIdx.y * 64;
+  const int t0 = ((int)gridDim.z - 1 - (int)blockIdx.z) * kSq;
+  const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int b = lane / 16, j = lane % 16, wx = wave % 2, wn = wave / 2;
+  const int nmax = min(a.pos0 + t0 + kSq, a.pos0 + a.T);  // positions of the last row
+  const int nc = (nmax + kPvCh - 1) / kPvCh;
+  const int kvh = h / (a.nq / a.nkv);
+  // instruction `wave` loads p rows (8 each), 4 + wave and 8 + wave V rows (4 each)
+  const int prow = 8 * wave + lane / PS, pcol = 4 * ((lane % PS) ^ ((prow >> 1) & 7));
+  const float* psrc = a.S + ((size_t)h * a.T + min(t0 + prow, a.T - 1)) * a.ss + pcol;
+  const float* vbase = a.vc + (size_t)kvh * a.max_seq * hd;
+  // V slot s of row r sits at s ^ 4 (r >> 2 & 3): the four blocks' rows 4b + c
+  // then meet four different quarters of the banks
+  int vrow[2], vcol[2];
+#pragma unroll
+  for (int v = 0; v < 2; ++v) {
+    vrow[v] = 4 * (wave + 4 * v) + lane / VS;
+    vcol[v] = d0 + 4 * ((lane % VS) ^ (4 * ((vrow[v] >> 2) & 3)));
+  }
+  auto load = [&](int c, int half) {
+    uint8_t* l = reinterpret_cast<uint8_t*>(lds4[half]);
+    const int c0 = c * kPvCh;
+    lds_load16(c0 + pcol < a.ss ? psrc + c0 : kDenseZero, l + wave * 1024);
+#pragma unroll
+    for (int v = 0; v < 2; ++v)
+      lds_load16(vcol[v] < hd ? vbase + (size_t)min(c0 + vrow[v], nmax - 1) * hd + vcol[v] : kDenseZero,
+                 l + (4 + wave + 4 * v) * 1024);
+  };
+  const int nlo = a.pos0 + t0 + 16 * wx + 1, nhi = nlo + 15;   // positions of the wave's rows
+  float acc[2][4] = {};
+  load(0, 0);
+  for (int c = 0; c < nc; ++c) {
+    stage_sync<0>();
+    if (c + 1 < nc) load(c + 1, (c + 1) & 1);
+    const float4* P = lds4[c & 1] + (16 * wx + j) * PS;
+    const float* V = reinterpret_cast<const float*>(lds4[c & 1] + kSq * PS);
+#pragma unroll
+    for (int g = 0; g < kPvCh / 16; ++g) {
+      const int pos = c * kPvCh + 16 * g;
+      if (pos >= nhi) break;
+      const float4 x = P[(4 * g + b) ^ ((j >> 1) & 7)];
+      float4 w[2];
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const float* v = V + (16 * g + 4 * b) * 64 + 4 * ((4 * (2 * wn + t) + j / 4) ^ (4 * b)) + j % 4;
+        w[t] = make_float4(v[0], v[64], v[128], v[192]);
+      }
+      const bool masked = pos + 16 > nlo;
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        v16f p[4];
+        mfma_products(x, w[t], p);
+        if (masked) {
+          int left = a.pos0 + t0 + 16 * wx + 4 * b + 1 - pos;   // row r: left + r positions from pos on
+          asm volatile("" : "+v"(left));   // (64 comparison masks kept for both tiles would spill)
+#pragma unroll
+          for (int k = 0; k < 16; ++k)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              const float q = p[k % 4][4 * (k / 4) + r];
+              p[k % 4][4 * (k / 4) + r] = k < left + r ? q : 0.0f;
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int k = 0; k < 16; ++k)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) acc[t][r] = acc[t][r] + p[k % 4][4 * (k / 4) + r];
+        __builtin_amdgcn_sched_barrier(0);
+      }
     }
   }
-  if (row_live && dd < dl) a.H[(size_t)(t0 + qi) * a.nq * hd + (size_t)h * hd + d0 + dd] = out;
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int tok = t0 + 16 * wx + 4 * b + r, d = d0 + 16 * (2 * wn + t) + j;
+      if (tok < a.T && d < hd) a.H[(size_t)tok * a.nq * hd + (size_t)h * hd + d] = acc[t][r];
+    }
 }
 
 // ---------------------------------------------------------------- misc
@@ -1786,7 +1908,11 @@ moe_status embed_rows(const int32_t* ids, int T, const float* emb, int V, int D,
 moe_status heads_norm_rope(const HeadArgs& a, hipStream_t s) {
   if (a.T <= 0) return MOE_OK;
   if (a.hd > kMaxHd || (a.hd & 1)) return set_error(MOE_ERR_ARG, "head_dim %d unsupported", a.hd);
-  hipLaunchKernelGGL(heads_kernel, dim3((unsigned)a.T, (unsigned)(a.nq + 2 * a.nkv)), dim3(64), 0, s, a);
+  const size_t lds = (size_t)2 * kHeadRows * (a.hd + 4) * 4;
+  moe_status st = set_lds(heads_kernel, lds, "heads LDS attribute");
+  if (st) return st;
+  const long long rows = (long long)a.T * (a.nq + 2 * a.nkv);
+  hipLaunchKernelGGL(heads_kernel, dim3((unsigned)((rows + kHeadRows - 1) / kHeadRows)), dim3(256), lds, s, a);
   return check_hip(hipGetLastError(), "heads launch");
 }
 
@@ -1794,25 +1920,25 @@ moe_status attention_rows(const AttnArgs& a, hipStream_t s) {
   if (a.T <= 0) return MOE_OK;
   if (a.hd % 4 || a.hd > kMaxHd) return set_error(MOE_ERR_ARG, "attention: head_dim %d", a.hd);
   if (a.fuse_heads && a.T != 1) return set_error(MOE_ERR_ARG, "attention: fused heads need T == 1");
-  if (a.T > 4 && !a.fuse_heads && a.nkv > 0 && a.nq % a.nkv == 0 &&
-      attn_pv_qt_lds(a.pos0, a.T) <= 160 * 1024 && !getenv("MOEHIP_ATTN_ROWWISE")) {
-    const unsigned qg = (unsigned)((a.T + kQt - 1) / kQt);
-    const size_t lds_s = ((size_t)64 * (a.hd + 4) + (size_t)kSq * a.hd) * 4;
+  if (a.T > 4 && !a.fuse_heads && a.nkv > 0 && a.nq % a.nkv == 0 && a.ss % 4 == 0 && al16(a.qkv) &&
+      a.ld % 4 == 0 && !getenv("MOEHIP_ATTN_ROWWISE")) {
+    const unsigned qg = (unsigned)((a.T + kSq - 1) / kSq);
+    const dim3 sg((unsigned)a.nq, (unsigned)((a.pos0 + a.T + kSk * kSkt - 1) / (kSk * kSkt)), qg);
+    const size_t lds_s = (size_t)((a.hd + 63) / 64 + kSkD) * kStageB;
     moe_status st;
     if ((st = set_lds(attn_scores_qt_kernel, lds_s, "scores LDS attribute"))) return st;
-    hipLaunchKernelGGL(attn_scores_qt_kernel,
-                       dim3((unsigned)((a.pos0 + a.T + 63) / 64), (unsigned)a.nq, (unsigned)((a.T + kSq - 1) / kSq)),
-                       dim3(256), lds_s, s, a);
+    hipLaunchKernelGGL(attn_scores_qt_kernel, sg, dim3(256), lds_s, s, a);
     if ((st = check_hip(hipGetLastError(), "scores launch"))) return st;
-    const size_t lds_m = attn_softmax_rows_lds(a.pos0, a.T);
+    // rows a block: 16, fewer where they would not fit two blocks a CU
+    int R = kSmRowsMax;
+    const size_t row_b = (size_t)sm_row_floats(a.pos0 + a.T) * 4;
+    while (R > 1 && R * row_b > 72 * 1024) R /= 2;
+    const size_t lds_m = R * row_b;
     if ((st = set_lds(attn_softmax_rows_kernel, lds_m, "softmax rows LDS attribute"))) return st;
-    hipLaunchKernelGGL(attn_softmax_rows_kernel, dim3((unsigned)((a.nq + kSmRowWaves - 1) / kSmRowWaves), (unsigned)a.T),
-                       dim3(kSmRowWaves * kWave), lds_m, s, a);
+    hipLaunchKernelGGL(attn_softmax_rows_kernel, dim3((unsigned)a.nq, (unsigned)((a.T + R - 1) / R)), dim3(256), lds_m,
+                       s, a, R);
     if ((st = check_hip(hipGetLastError(), "softmax rows launch"))) return st;
-    const size_t lds_p = attn_pv_qt_lds(a.pos0, a.T);
-    if ((st = set_lds(attn_pv_qt_kernel, lds_p, "softmax/pv LDS attribute"))) return st;
-    hipLaunchKernelGGL(attn_pv_qt_kernel, dim3((unsigned)((a.hd + kPvDpb - 1) / kPvDpb), (unsigned)a.nq, qg),
-                       dim3(256), lds_p, s, a);
+    hipLaunchKernelGGL(attn_pv_qt_kernel, dim3((unsigned)a.nq, (unsigned)((a.hd + 63) / 64), qg), dim3(256), 0, s, a);
     return check_hip(hipGetLastError(), "softmax/pv launch");
   }
   const int nmax = a.pos0 + a.T;   // positions of the last row

@@ -131,6 +131,10 @@ void free_model(moe_model* m) {
   delete m;
 }
 
+// Floats between two score rows: whole 16-byte loads, and an odd number of
+// 256-byte pieces, so that neighbouring rows start in different cache channels.
+int score_stride(const moe_model* m) { return 64 * ((m->max_seq + 63) / 64 | 1); }
+
 moe_status check_cfg(const QwenConfig* c, int max_seq) {
   if (c->d_model <= 0 || c->n_layers <= 0 || c->head_dim <= 0 || c->n_q <= 0 || c->n_kv <= 0 ||
       c->d_ff <= 0 || c->n_experts <= 0 || c->top_k <= 0 || c->vocab_size <= 0)
@@ -189,7 +193,7 @@ moe_status ensure_scratch(moe_model* m, int T) {
   const size_t td = (size_t)T * c.d_model * 4;
   if ((st = grow(m->x, td)) || (st = grow(m->xa, td)) || (st = grow(m->xn, td)) ||
       (st = grow(m->qkv, (size_t)T * m->nqkv * 4)) || (st = grow(m->H, (size_t)T * m->Dq * 4)) ||
-      (st = grow(m->S, (size_t)T * c.n_q * m->max_seq * 4)) || (st = grow(m->ids, (size_t)T * 4)))
+      (st = grow(m->S, (size_t)T * c.n_q * score_stride(m) * 4)) || (st = grow(m->ids, (size_t)T * 4)))
     return st;
   return MOE_OK;
 }
@@ -225,7 +229,7 @@ moe_status forward_dev(moe_model* m, const int32_t* ids_d, int T, float* logits_
     // :371-398 q/k norm, :400 RoPE, K/V into the cache
     // (one token: done inside the score launch)
     AttnArgs aa{qkv, m->nqkv, kc, vc, (float*)m->S.p, (float*)m->H.p, T, m->pos, c.n_q, c.n_kv,
-                hd, m->max_seq, m->scale};
+                hd, m->max_seq, score_stride(m), m->scale};
     if (T == 1) {
       aa.fuse_heads = 1;
       aa.q_norm = L.q_norm; aa.k_norm = L.k_norm; aa.eps = eps;
