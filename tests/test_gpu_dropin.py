@@ -1,0 +1,64 @@
+"""The drop-in matmul_adaptive on weights it has seen before: the product
+starts on the cached device copy while the host bytes are checked, so a weight
+changed in place must still give the new weights' result, bit for bit."""
+import numpy as np
+import pytest
+
+import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def bits(a):
+    return np.ascontiguousarray(a, dtype=np.float32).view(np.uint32)
+
+
+def want_of(dtype, A, w, s, N, K):
+    if dtype == 0:
+        return O.matmul_f32(A, w)
+    return (O.gemv_q8 if dtype == 2 else O.gemv_q4)(A, w, s, N, K)
+
+
+# (dtype, M, N, K): C stored straight into pinned memory, C just past 64 KB
+# (copied), C past 1 MB and A past 1 MB (no pinned staging); weight bytes a
+# multiple of the digest's 128-byte block and not
+CASES = [(2, 1, 768, 2048), (3, 2, 70, 98), (0, 3, 33, 68), (2, 3, 6000, 64), (3, 40, 8000, 64),
+         (0, 300, 20, 1000), (2, 1, 1, 130)]
+
+
+@pytest.mark.parametrize("dtype,M,N,K", CASES)
+def test_dropin_weights_changed_in_place(moehip, dtype, M, N, K):
+    print("drop-in case", dtype, M, N, K, flush=True)
+    A = O.normal(M * K, 5, 0.0, 1.0).reshape(M, K)
+    if dtype == 0:
+        w, s = O.normal(N * K, 6, 0.0, 0.05).reshape(N, K), None
+    else:
+        w, s = (O.quant_q8 if dtype == 2 else O.quant_q4)(O.normal(N * K, 6, 0.0, 0.02).reshape(N, K))
+
+    def call():
+        if dtype == 0:
+            return moehip.matmul_adaptive(A, w, None, N, K)
+        return moehip.matmul_adaptive(A, None, {"q": w, "s": s, "dtype": dtype}, N, K)
+
+    for _ in range(2):
+        np.testing.assert_array_equal(bits(call()), bits(want_of(dtype, A, w, s, N, K)))
+    raw = w.reshape(-1).view(np.uint8)
+    for at in (0, raw.size // 2, raw.size - 1):
+        raw[at] ^= 0x11     # (an fp32 weight keeps its exponent: bits of the mantissa or of its low byte)
+        for _ in range(2):
+            np.testing.assert_array_equal(bits(call()), bits(want_of(dtype, A, w, s, N, K)))
+    if s is not None:
+        s[N - 1] *= np.float32(1.5)
+        np.testing.assert_array_equal(bits(call()), bits(want_of(dtype, A, w, s, N, K)))
+    # trusted addresses keep the last upload; verified again, the change is seen
+    L = moehip.lib()
+    old = want_of(dtype, A, w, s, N, K)
+    moehip.check(L.moe_weight_cache_mode(1))
+    raw[3] ^= 0x11
+    try:
+        np.testing.assert_array_equal(bits(call()), bits(old))
+    finally:
+        moehip.check(L.moe_weight_cache_mode(0))
+    np.testing.assert_array_equal(bits(call()), bits(want_of(dtype, A, w, s, N, K)))
+    moehip.check(L.moe_weight_cache_clear())
+    np.testing.assert_array_equal(bits(call()), bits(want_of(dtype, A, w, s, N, K)))
