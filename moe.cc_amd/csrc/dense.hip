@@ -109,6 +109,17 @@ __global__ __launch_bounds__(64 * (NP + 1)) void dense_gemv_kernel(DenseArgs a) 
   constexpr int NW = RW / RPL;               // W float4 per producer lane per chunk
   constexpr int NB = NP + 1;                 // LDS product buffers
   constexpr int NT = 64 * (NP + 1);
+  if constexpr (RW == 1) {   // tokens 16 blockIdx.y .. (17-32 given rows: two groups)
+    const int m0 = MM * (int)blockIdx.y;
+    a.M = min(a.M - m0, MM);
+    a.A += (size_t)m0 * a.lda;
+    a.C += (size_t)m0 * a.ldc;
+    if (a.resid) a.resid += (size_t)m0 * a.ldr;
+    if constexpr (PACK != 0) {
+      a.pack_tabs += (size_t)m0 * act_table_bytes(a.K);
+      a.pack_part += (size_t)blockIdx.y * gridDim.x * 16 * 2;
+    }
+  }
   extern __shared__ float4 pl4[];
   float* pl = reinterpret_cast<float*>(pl4);
   __shared__ float inv_s[MM];
@@ -1720,11 +1731,12 @@ size_t gemv_lds(int RW, int NP, int M, int K, bool norm) {
 
 template <int RW, bool NORM, int PACK, int NP, int MMX = 64 / RW>
 moe_status launch_gemv(const DenseArgs& a, hipStream_t s) {
-  const size_t lds = gemv_lds(RW, NP, a.M, a.K, NORM);
+  const int groups = RW == 1 ? (a.M + MMX - 1) / MMX : 1;
+  const size_t lds = gemv_lds(RW, NP, groups > 1 ? MMX : a.M, a.K, NORM);
   moe_status st = set_lds(dense_gemv_kernel<RW, NORM, PACK, NP, MMX>, lds, "gemv LDS attribute");
   if (st) return st;
-  hipLaunchKernelGGL((dense_gemv_kernel<RW, NORM, PACK, NP, MMX>), dim3((unsigned)((a.N + RW - 1) / RW)),
-                     dim3(64 * (NP + 1)), lds, s, a);
+  hipLaunchKernelGGL((dense_gemv_kernel<RW, NORM, PACK, NP, MMX>),
+                     dim3((unsigned)((a.N + RW - 1) / RW), (unsigned)groups), dim3(64 * (NP + 1)), lds, s, a);
   return check_hip(hipGetLastError(), "dense gemv launch");
 }
 
@@ -1763,16 +1775,22 @@ bool dense_row_ok(const DenseArgs& a, bool vec) {
   return rows && a.N <= 1024 && vec && a.K <= kRowMaxK && !a.amax_part;
 }
 
-bool dense_rows4_ok(const DenseArgs& a, bool vec) {
-  return a.M > 4 && a.M <= 16 && !a.norm && !a.sel_counter && !a.amax_part && a.N <= 1024 && vec &&
-         a.K <= kRowsMaxK;
-}
-
 // The block-parallel rows kernel instead of the chain kernel for 5-16
 // given rows (MOEHIP_ROUTER_ROWS4=1, for comparison).
 bool rows4_kernel_chosen() {
   static const bool v = getenv("MOEHIP_ROUTER_ROWS4") != nullptr;
   return v;
+}
+
+// Given rows against few rows (the router): 5-16 on either rows kernel, 17-32
+// against up to 256 rows (one round of blocks) on the chain kernel as two
+// groups of blocks, where the 32 x 32 MFMA tiles run on a few CUs and the
+// packing takes a launch of its own (Q8 layer of 20 tokens 209 -> 127 us, Q4
+// 162 -> 79).
+bool dense_rows4_ok(const DenseArgs& a, bool vec) {
+  if (a.M > 16 && (a.M > 32 || a.N > 256 || rows4_kernel_chosen())) return false;
+  return a.M > 4 && !a.norm && !a.sel_counter && !a.amax_part && a.N <= 1024 && vec &&
+         a.K <= kRowsMaxK;
 }
 
 bool dense_rows4_path(const DenseArgs& a) {

@@ -640,7 +640,7 @@ moe_status ensure_scratch(LayerDev* L, int T) {
       (st = grow(S.htab, np * act_table_bytes(L->dff), &synced)) ||
       (st = grow(S.h, np * L->dff * 4, &synced)) || (st = grow(S.xn, (size_t)T * L->D * 4, &synced)) ||
       (st = grow(S.hpart, np * (size_t)((L->dff + 7) / 8) * 8, &synced)) ||
-      (st = grow(S.xpart, (size_t)(T > 4 ? 16 : T) * (L->E + 16) * 8, &synced)))
+      (st = grow(S.xpart, (size_t)(T > 16 ? 32 : T > 4 ? 16 : T) * (L->E + 16) * 8, &synced)))
     return st;
   if (grouped_ok(L) &&
       ((st = grow(S.ecount, (size_t)L->E * 4, &synced)) || (st = grow(S.eoff, (size_t)L->E * 4, &synced)) ||
@@ -928,8 +928,9 @@ moe_status layer_forward_run(LayerDev* L, const float* x, float norm_eps, const 
   } else if (fuse_sel && T <= 4 && dense_row_path(ra)) {
     // up to four given rows: the router's row kernel packs the x tables too
     ra.pack_dtype = L->dtype; ra.pack_tabs = L->xtab; ra.pack_part = L->xpart;
-  } else if (!fuse_sel && dense_rows4_path(ra)) {
-    // 5-16 given rows: the router's rows kernel packs the x tables too, the
+  } else if (!fuse_sel && (T <= 16 || allow_grouped) && dense_rows4_path(ra)) {
+    // 5-32 given rows (16 with the no-allocation scratch, whose partials hold
+    // one token group): the router's rows kernel packs the x tables too, the
     // selection kernel writes their headers
     ra.pack_dtype = L->dtype; ra.pack_tabs = L->xtab; ra.pack_part = L->xpart;
   } else {
