@@ -544,28 +544,48 @@ __global__ __launch_bounds__(kTileBlock) void gate_up_down_kernel(FuseArgs f) {
 
 // rmsnorm (test_model_trace.c:241-255): one block per token; the squares
 // x_i * x_i are formed by all threads into LDS and summed in order by
-// block_seq_sum (msq / D, 1 / sqrtf(msq + eps)).
-__global__ __launch_bounds__(256) void rmsnorm_kernel(const float* __restrict__ x,
-                                                      const float* __restrict__ w,
-                                                      float* __restrict__ y, int D, float eps,
-                                                      int fast) {
+// block_seq_sum (msq / D, 1 / sqrtf(msq + eps)).  Latency: 512 threads give
+// each candidate chain of the sum a thread of its own, and a row of up to 2048
+// columns is read once (5 tokens 7.5 -> 4.6 us, 512 tokens 8.7 -> 6.6).
+constexpr int kRmsThreads = 512;
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+
+__global__ __launch_bounds__(kRmsThreads) void rmsnorm_kernel(const float* __restrict__ x,
+                                                              const float* __restrict__ w,
+                                                              float* __restrict__ y, int D, float eps,
+                                                              int fast) {
   extern __shared__ float4 sq4[];
   __shared__ float inv_s;
   __shared__ SeqSumScratch seq;
-  const int t = blockIdx.x;
+  const int t = blockIdx.x, tid = threadIdx.x;
   const float* xt = x + (size_t)t * D;
   if (fast) {
-    for (int i = threadIdx.x; i < D / 4; i += blockDim.x) {
+    // the row's first float4 a thread and its weights stay in registers
+    const bool in0 = tid < D / 4;
+    const float4 v0 = in0 ? reinterpret_cast<const float4*>(xt)[tid] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    f32x4_any w0 = {1.0f, 1.0f, 1.0f, 1.0f};
+    if (in0 && w) w0 = reinterpret_cast<const f32x4_any*>(w)[tid];
+    if (in0) sq4[tid] = make_float4(v0.x * v0.x, v0.y * v0.y, v0.z * v0.z, v0.w * v0.w);
+    for (int i = tid + kRmsThreads; i < D / 4; i += kRmsThreads) {
       const float4 v = reinterpret_cast<const float4*>(xt)[i];
       sq4[i] = make_float4(v.x * v.x, v.y * v.y, v.z * v.z, v.w * v.w);
     }
     __syncthreads();
-    const float acc = block_seq_sum<256>(reinterpret_cast<const float*>(sq4), D, seq);
-    if (threadIdx.x == 0) {
-      const float msq = acc / (float)D;
-      inv_s = 1.0f / sqrtf(msq + eps);
+    const float acc = block_seq_sum<kRmsThreads>(reinterpret_cast<const float*>(sq4), D, seq);
+    const float inv = 1.0f / sqrtf(acc / (float)D + eps);
+    float* yt = y + (size_t)t * D;
+    if (in0) {
+      const float n0 = v0.x * inv, n1 = v0.y * inv, n2 = v0.z * inv, n3 = v0.w * inv;
+      const f32x4_any o = {n0 * w0[0], n1 * w0[1], n2 * w0[2], n3 * w0[3]};
+      reinterpret_cast<f32x4_any*>(yt)[tid] = o;
     }
-  } else if (threadIdx.x == 0) {
+    for (int i = 4 * kRmsThreads + tid; i < D; i += kRmsThreads) {
+      const float v = xt[i] * inv;
+      yt[i] = v * (w ? w[i] : 1.0f);
+    }
+    return;
+  }
+  if (tid == 0) {
     float msq = 0.0f;
     for (int i = 0; i < D; ++i) {
       const float sq = xt[i] * xt[i];
@@ -576,7 +596,7 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(const float* __restrict__ 
   }
   __syncthreads();
   const float inv = inv_s;
-  for (int i = threadIdx.x; i < D; i += blockDim.x) {
+  for (int i = tid; i < D; i += kRmsThreads) {
     const float v = xt[i] * inv;
     y[(size_t)t * D + i] = v * (w ? w[i] : 1.0f);
   }
@@ -1082,7 +1102,7 @@ moe_status rmsnorm_dev(const float* x, const float* w, float* y, int T, int D, f
                                                   (int)lds), "rmsnorm LDS attribute");
     if (st) return st;
   }
-  hipLaunchKernelGGL(rmsnorm_kernel, dim3(T), dim3(256), lds, stream(), x, w, y, D, eps, fast);
+  hipLaunchKernelGGL(rmsnorm_kernel, dim3(T), dim3(kRmsThreads), lds, stream(), x, w, y, D, eps, fast);
   return check_hip(hipGetLastError(), "rmsnorm launch");
 }
 
