@@ -76,7 +76,7 @@ def test_c_caller_compiles_and_links():
     assert {"matmul_adaptive", "moe_layer_create", "moe_layer_forward"} <= undef
 
 
-@pytest.mark.skipif(not (os.path.exists(LIB) and os.path.isdir("/root/reference")),
+@pytest.mark.skipif(not (os.path.exists(LIB) and os.path.isfile("/root/reference/kernels.c")),
                     reason="needs libmoehip.so and the reference tree (build container only)")
 def test_reference_links_against_library():
     """INTEGRATION.md's relink: the reference's own test_model_trace.o, io.o
