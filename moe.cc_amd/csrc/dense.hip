@@ -657,8 +657,16 @@ __device__ __forceinline__ void mfma_products(const float4& x, const float4& w, 
 
 __device__ __align__(16) const float kDenseZero[4] = {};
 
-template <int WX, int NB, int KC, int D>
-__global__ __launch_bounds__(256, 4) void dense_mfma_kernel(DenseArgs a) {
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+
+// ANY: rows of any length at any 4-byte alignment, which the direct loads to
+// LDS do not take: each lane's 16 bytes of the next chunk go through registers
+// while the chunk before is multiplied (two LDS buffers).  Against a thread an
+// output (dense_generic_kernel, bound by its uncoalesced row reads): 1 x 8192 x
+// 4095 1822 -> 65 us, 7 x 3000 x 1001 288 -> 19, 100 x 2048 x 4095 1522 -> 64,
+// 512 x 5120 x 2047 20.9 ms -> 258 us.
+template <int WX, int NB, int KC, int D, bool ANY>
+__global__ __launch_bounds__(256, ANY ? 3 : 4) void dense_mfma_kernel(DenseArgs a) {
   constexpr int WN = 4 / WX;
   constexpr int RX = 16 * WX, RW = 16 * NB * WN, R = RX + RW;
   constexpr int SL = KC / 4;                 // 16-byte slots of an LDS row
@@ -681,9 +689,30 @@ __global__ __launch_bounds__(256, 4) void dense_mfma_kernel(DenseArgs a) {
   for (int v = 0; v < NL; ++v) {
     const int row = RPI * ((wave + 4 * v) % NI) + lane / SL;   // past the tile: another wave's rows again
     col[v] = 4 * ((lane % SL) ^ sw(row));
-    src[v] = row < RX ? a.A + (size_t)min(t0 + row, a.M - 1) * a.lda + col[v]
-                      : a.W + (size_t)min(n0 + row - RX, a.N - 1) * a.ldw + col[v];
+    src[v] = row < RX ? a.A + (size_t)min(t0 + row, a.M - 1) * a.lda + (ANY ? 0 : col[v])
+                      : a.W + (size_t)min(n0 + row - RX, a.N - 1) * a.ldw + (ANY ? 0 : col[v]);
   }
+  f32x4_any next[ANY ? NL : 1];
+  auto fetch = [&](int c) {
+    if ((c + 1) * KC <= a.K) {
+#pragma unroll
+      for (int v = 0; v < NL; ++v) next[v] = *reinterpret_cast<const f32x4_any*>(src[v] + c * KC + col[v]);
+    } else {   // columns past K: the row's last one read again, zero taken
+#pragma unroll
+      for (int v = 0; v < NL; ++v)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int k = c * KC + col[v] + e;
+          const float f = src[v][min(k, a.K - 1)];
+          next[v][e] = k < a.K ? f : 0.0f;
+        }
+    }
+  };
+  auto store = [&](int h) {
+#pragma unroll
+    for (int v = 0; v < NL; ++v)
+      lds4[h][((wave + 4 * v) % NI) * 64 + lane] = make_float4(next[v][0], next[v][1], next[v][2], next[v][3]);
+  };
   auto load = [&](int c, int h) {
     uint8_t* l = reinterpret_cast<uint8_t*>(lds4[h]);
     if ((c + 1) * KC <= a.K) {
@@ -702,10 +731,22 @@ __global__ __launch_bounds__(256, 4) void dense_mfma_kernel(DenseArgs a) {
   for (int t = 0; t < NB; ++t)
 #pragma unroll
     for (int r = 0; r < 4; ++r) acc[t][r] = 0.0f;
-  for (int p = 0; p < D - 1; ++p) load(min(p, nc - 1), p);
+  static_assert(!ANY || D == 2, "the register path alternates two buffers");
+  if constexpr (ANY) {
+    fetch(0);
+    store(0);
+  } else {
+    for (int p = 0; p < D - 1; ++p) load(min(p, nc - 1), p);
+  }
+#pragma unroll 1
   for (int c = 0; c < nc; ++c) {
-    stage_sync<(D - 2) * NL>();
-    load(min(c + D - 1, nc - 1), (c + D - 1) % D);
+    if constexpr (ANY) {
+      __syncthreads();   // chunk c is in LDS, every wave is done with chunk c - 1
+      fetch(min(c + 1, nc - 1));
+    } else {
+      stage_sync<(D - 2) * NL>();
+      load(min(c + D - 1, nc - 1), (c + D - 1) % D);
+    }
     const float4* B = lds4[c % D] + j * SL;
     constexpr int STEPS = KC / 16 * NB;   // 16 columns of one row tile each
     auto read_x = [&](int g) { return B[16 * wx * SL + ((4 * g + b) ^ sw(j))]; };
@@ -731,8 +772,14 @@ __global__ __launch_bounds__(256, 4) void dense_mfma_kernel(DenseArgs a) {
       x = xn;
       w = wn4;
     }
+    if constexpr (ANY) {
+#pragma unroll
+      for (int t = 0; t < NB; ++t)   // the adds stay before the store
+        asm volatile("" : "+v"(acc[t][0]), "+v"(acc[t][1]), "+v"(acc[t][2]), "+v"(acc[t][3]));
+      store((c + 1) % D);
+    }
   }
-  stage_sync<0>();   // the clamped loads past the last chunk have landed
+  if constexpr (!ANY) stage_sync<0>();   // the clamped loads past the last chunk have landed
 #pragma unroll
   for (int t = 0; t < NB; ++t)
 #pragma unroll
@@ -742,7 +789,8 @@ __global__ __launch_bounds__(256, 4) void dense_mfma_kernel(DenseArgs a) {
     }
 }
 
-// Any shape or alignment: one thread per output, plain loads.
+// Any shape or alignment: one thread per output, plain loads (more rows than a
+// grid of tiles takes).
 __global__ __launch_bounds__(256) void dense_generic_kernel(DenseArgs a) {
   const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
   if (i >= (long long)a.M * a.N) return;
@@ -1688,11 +1736,11 @@ moe_status set_lds(F* fn, size_t bytes, const char* what) {
   return st;
 }
 
-template <int WX, int NB, int KC, int D>
+template <int WX, int NB, int KC, int D, bool ANY>
 moe_status launch_mfma(const DenseArgs& a, hipStream_t s) {
   constexpr int RX = 16 * WX, RW = 16 * NB * (4 / WX);
   dim3 grid((unsigned)((a.N + RW - 1) / RW), (unsigned)((a.M + RX - 1) / RX));
-  hipLaunchKernelGGL((dense_mfma_kernel<WX, NB, KC, D>), grid, dim3(256), 0, s, a);
+  hipLaunchKernelGGL((dense_mfma_kernel<WX, NB, KC, D, ANY>), grid, dim3(256), 0, s, a);
   return check_hip(hipGetLastError(), "dense mfma launch");
 }
 
@@ -1704,6 +1752,7 @@ moe_status launch_mfma(const DenseArgs& a, hipStream_t s) {
 // 64 x 64 116, 160, 246, 586 for m = 1, 2, 3, 8; 64 x 80 145, 199, 305 for m =
 // 1, 2, 3.  Small tiles spread few tokens over the CUs, large ones spend less
 // on operands per product.
+template <bool ANY>
 moe_status launch_mfma_best(const DenseArgs& a, hipStream_t s) {
   struct Shape { int rx, rw, step, odd; };
   static const Shape shapes[4] = {{32, 32, 22, 10}, {32, 64, 40, 18}, {64, 64, 75, 42}, {64, 80, 95, 50}};
@@ -1717,10 +1766,10 @@ moe_status launch_mfma_best(const DenseArgs& a, hipStream_t s) {
     if (i == 0 || t < tbest) { best = i; tbest = t; }
   }
   switch (best) {
-    case 0: return launch_mfma<2, 1, 64, 2>(a, s);
-    case 1: return launch_mfma<2, 2, 32, 2>(a, s);
-    case 2: return launch_mfma<4, 4, 32, 2>(a, s);
-    default: return launch_mfma<4, 5, 32, 2>(a, s);
+    case 0: return launch_mfma<2, 1, 64, 2, ANY>(a, s);
+    case 1: return launch_mfma<2, 2, 32, 2, ANY>(a, s);
+    case 2: return launch_mfma<4, 4, 32, 2, ANY>(a, s);
+    default: return launch_mfma<4, 5, 32, 2, ANY>(a, s);
   }
 }
 
@@ -1855,6 +1904,7 @@ moe_status dense_matmul(const DenseArgs& a, hipStream_t s) {
     if (a.pack_dtype == 3) return launch_gemv<16, true, 3, 1>(a, s);
     return launch_gemv<16, true, 0, 1>(a, s);
   }
+  if (!vec && (a.M + 31) / 32 <= 65535) return launch_mfma_best<true>(a, s);
   if (!vec) {
     const long long total = (long long)a.M * a.N;
     hipLaunchKernelGGL(dense_generic_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, a);
@@ -1912,7 +1962,7 @@ moe_status dense_matmul(const DenseArgs& a, hipStream_t s) {
     // tiles are never slower (16 x 1100 x 1024: 21 against 16)
     return launch_gemv<4, false, 0, 1>(a, s);
   } else {
-    return launch_mfma_best(a, s);
+    return launch_mfma_best<false>(a, s);
   }
 }
 
