@@ -663,10 +663,11 @@ typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
 // LDS do not take: each lane's 16 bytes of the next chunk go through registers
 // while the chunk before is multiplied (two LDS buffers).  Against a thread an
 // output (dense_generic_kernel, bound by its uncoalesced row reads): 1 x 8192 x
-// 4095 1822 -> 65 us, 7 x 3000 x 1001 288 -> 19, 100 x 2048 x 4095 1522 -> 64,
-// 512 x 5120 x 2047 20.9 ms -> 258 us.
+// 4095 1822 -> 64 us, 7 x 3000 x 1001 288 -> 18, 100 x 2048 x 4095 1522 -> 64,
+// 512 x 5120 x 2047 20.9 ms -> 179 us (the direct loads at K = 2048: 170).  The
+// two large tiles spill at four waves a SIMD: 247 us there, 179 at three.
 template <int WX, int NB, int KC, int D, bool ANY>
-__global__ __launch_bounds__(256, ANY ? 3 : 4) void dense_mfma_kernel(DenseArgs a) {
+__global__ __launch_bounds__(256, ANY && NB >= 4 ? 3 : 4) void dense_mfma_kernel(DenseArgs a) {
   constexpr int WN = 4 / WX;
   constexpr int RX = 16 * WX, RW = 16 * NB * WN, R = RX + RW;
   constexpr int SL = KC / 4;                 // 16-byte slots of an LDS row
@@ -693,22 +694,23 @@ __global__ __launch_bounds__(256, ANY ? 3 : 4) void dense_mfma_kernel(DenseArgs 
                       : a.W + (size_t)min(n0 + row - RX, a.N - 1) * a.ldw + (ANY ? 0 : col[v]);
   }
   f32x4_any next[ANY ? NL : 1];
+  // K >= 4: a load that would pass the row's end is moved back to end with it,
+  // and its columns moved down (zeros from K on) on the way to LDS
   auto fetch = [&](int c) {
-    if ((c + 1) * KC <= a.K) {
 #pragma unroll
-      for (int v = 0; v < NL; ++v) next[v] = *reinterpret_cast<const f32x4_any*>(src[v] + c * KC + col[v]);
-    } else {   // columns past K: the row's last one read again, zero taken
-#pragma unroll
-      for (int v = 0; v < NL; ++v)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int k = c * KC + col[v] + e;
-          const float f = src[v][min(k, a.K - 1)];
-          next[v][e] = k < a.K ? f : 0.0f;
-        }
-    }
+    for (int v = 0; v < NL; ++v)
+      next[v] = *reinterpret_cast<const f32x4_any*>(src[v] + min(c * KC + col[v], a.K - 4));
   };
-  auto store = [&](int h) {
+  auto store = [&](int c, int h) {
+    if ((c + 1) * KC > a.K) {
+#pragma unroll
+      for (int v = 0; v < NL; ++v) {
+        const int d = c * KC + col[v] - min(c * KC + col[v], a.K - 4);
+        if (d & 1) next[v] = f32x4_any{next[v][1], next[v][2], next[v][3], 0.0f};
+        if (d & 2) next[v] = f32x4_any{next[v][2], next[v][3], 0.0f, 0.0f};
+        if (d >= 4) next[v] = f32x4_any{0.0f, 0.0f, 0.0f, 0.0f};
+      }
+    }
 #pragma unroll
     for (int v = 0; v < NL; ++v)
       lds4[h][((wave + 4 * v) % NI) * 64 + lane] = make_float4(next[v][0], next[v][1], next[v][2], next[v][3]);
@@ -734,7 +736,7 @@ __global__ __launch_bounds__(256, ANY ? 3 : 4) void dense_mfma_kernel(DenseArgs 
   static_assert(!ANY || D == 2, "the register path alternates two buffers");
   if constexpr (ANY) {
     fetch(0);
-    store(0);
+    store(0, 0);
   } else {
     for (int p = 0; p < D - 1; ++p) load(min(p, nc - 1), p);
   }
@@ -768,15 +770,14 @@ __global__ __launch_bounds__(256, ANY ? 3 : 4) void dense_mfma_kernel(DenseArgs 
       for (int k = 0; k < 16; ++k)
 #pragma unroll
         for (int r = 0; r < 4; ++r) acc[t][r] = acc[t][r] + p[k % 4][4 * (k / 4) + r];
+      if constexpr (ANY)   // the adds stay here, not sunk towards the store
+        asm volatile("" : "+v"(acc[t][0]), "+v"(acc[t][1]), "+v"(acc[t][2]), "+v"(acc[t][3]));
       __builtin_amdgcn_sched_barrier(0);
       x = xn;
       w = wn4;
     }
     if constexpr (ANY) {
-#pragma unroll
-      for (int t = 0; t < NB; ++t)   // the adds stay before the store
-        asm volatile("" : "+v"(acc[t][0]), "+v"(acc[t][1]), "+v"(acc[t][2]), "+v"(acc[t][3]));
-      store((c + 1) % D);
+      store(min(c + 1, nc - 1), (c + 1) % D);
     }
   }
   if constexpr (!ANY) stage_sync<0>();   // the clamped loads past the last chunk have landed
@@ -789,8 +790,8 @@ __global__ __launch_bounds__(256, ANY ? 3 : 4) void dense_mfma_kernel(DenseArgs 
     }
 }
 
-// Any shape or alignment: one thread per output, plain loads (more rows than a
-// grid of tiles takes).
+// Any shape or alignment: one thread per output, plain loads (rows under
+// four columns, more rows than a grid of tiles takes).
 __global__ __launch_bounds__(256) void dense_generic_kernel(DenseArgs a) {
   const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
   if (i >= (long long)a.M * a.N) return;
@@ -1904,7 +1905,7 @@ moe_status dense_matmul(const DenseArgs& a, hipStream_t s) {
     if (a.pack_dtype == 3) return launch_gemv<16, true, 3, 1>(a, s);
     return launch_gemv<16, true, 0, 1>(a, s);
   }
-  if (!vec && (a.M + 31) / 32 <= 65535) return launch_mfma_best<true>(a, s);
+  if (!vec && a.K >= 4 && (a.M + 31) / 32 <= 65535) return launch_mfma_best<true>(a, s);
   if (!vec) {
     const long long total = (long long)a.M * a.N;
     hipLaunchKernelGGL(dense_generic_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, a);
