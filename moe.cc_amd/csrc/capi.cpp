@@ -2,8 +2,8 @@
 //
 // Library state: one device, one stream (default priority), a cache of
 // weights uploaded by the drop-in matmul_adaptive, a thread-local last-error
-// message.  Every entry point is thread-compatible; the cache is guarded by a
-// mutex.
+// message.  Every entry point is thread-compatible; the drop-in's calls from
+// several threads run one after another (g_dropin_mu).
 #include <hip/hip_runtime.h>
 
 #include <cstdarg>
@@ -24,8 +24,13 @@ namespace moe {
 
 namespace {
 thread_local std::string g_err;
+// Held for a whole matmul_adaptive call (its staging buffers and the cached
+// weights its launches read belong to one call at a time) and by whatever
+// frees those; taken before g_mu, which guards the library state and the
+// cache's map.
+std::mutex g_dropin_mu;
 std::mutex g_mu;
-bool g_ready = false;
+std::atomic<bool> g_ready{false};
 int g_device = -1;
 hipStream_t g_stream = nullptr;
 
@@ -162,8 +167,8 @@ moe_status cached_upload(const void* host, size_t bytes, const void** dev) {
   return MOE_OK;
 }
 
-// The cached device copy of a host weight, its content not yet checked
-// (moe_weight_cache_clear and another thread's upload aside, it stays).
+// The cached device copy of a host weight, its content not yet checked; it
+// stays while g_dropin_mu is held.
 bool cached_lookup(const void* host, size_t bytes, CacheEntry* e) {
   std::lock_guard<std::mutex> lk(g_mu);
   auto it = g_cache.find(CacheKey{host, bytes});
@@ -224,6 +229,7 @@ moe_status moe_synchronize(void) {
 }
 
 moe_status moe_weight_cache_clear(void) {
+  std::lock_guard<std::mutex> call(g_dropin_mu);
   moe_status st = ensure_init();
   if (st) return st;
   st = check_hip(hipStreamSynchronize(g_stream), "hipStreamSynchronize");
@@ -234,6 +240,7 @@ moe_status moe_weight_cache_clear(void) {
 }
 
 moe_status moe_weight_cache_mode(int trust_addresses) {
+  std::lock_guard<std::mutex> call(g_dropin_mu);
   std::lock_guard<std::mutex> lk(g_mu);
   g_trust_addresses = trust_addresses ? 1 : 0;
   return MOE_OK;
@@ -522,6 +529,7 @@ static moe_status dropin_enqueue(const float* A, int dtype, const void* dw, cons
 
 void matmul_adaptive(const float* A, const float* W_fp32, const void* W_q_ptr, float* C, int M,
                      int N, int K) {
+  std::lock_guard<std::mutex> call(g_dropin_mu);
   if (ensure_init()) die("matmul_adaptive init");
   if (M <= 0 || N <= 0) return;
   if (K < 0) K = 0;
@@ -578,6 +586,7 @@ void matmul_adaptive(const float* A, const float* W_fp32, const void* W_q_ptr, f
 }
 
 moe_status moe_shutdown(void) {
+  std::lock_guard<std::mutex> call(g_dropin_mu);
   std::lock_guard<std::mutex> lk(g_mu);
   if (!g_ready) return MOE_OK;
   const int live = g_live.load();

@@ -1,6 +1,8 @@
 """The drop-in matmul_adaptive on weights it has seen before: the product
 starts on the cached device copy while the host bytes are checked, so a weight
 changed in place must still give the new weights' result, bit for bit."""
+import threading
+
 import numpy as np
 import pytest
 
@@ -62,3 +64,37 @@ def test_dropin_weights_changed_in_place(moehip, dtype, M, N, K):
     np.testing.assert_array_equal(bits(call()), bits(want_of(dtype, A, w, s, N, K)))
     moehip.check(L.moe_weight_cache_clear())
     np.testing.assert_array_equal(bits(call()), bits(want_of(dtype, A, w, s, N, K)))
+
+
+def test_dropin_calls_from_several_threads(moehip):
+    """Calls on different operands from three host threads (C within 64 KB, C
+    past it, operands past the pinned staging) while a fourth clears the
+    weight cache: every result is its own call's."""
+    print("drop-in threads", flush=True)
+    work = []
+    for i, (dtype, M, N, K) in enumerate([(2, 1, 768, 2048), (3, 8, 4000, 256), (2, 130, 2100, 96)]):
+        A = O.normal(M * K, 31 + i, 0.0, 1.0).reshape(M, K)
+        w, s = (O.quant_q8 if dtype == 2 else O.quant_q4)(O.normal(N * K, 41 + i, 0.0, 0.02).reshape(N, K))
+        work.append((A, {"q": w, "s": s, "dtype": dtype}, N, K, want_of(dtype, A, w, s, N, K)))
+    wrong, left = [], [len(work)]
+    done = threading.Event()
+
+    def caller(i):
+        A, w, N, K, want = work[i]
+        try:
+            for it in range(40):
+                if not np.array_equal(bits(moehip.matmul_adaptive(A, None, w, N, K)), bits(want)):
+                    wrong.append((i, it))
+        finally:
+            left[0] -= 1
+            if not left[0]:
+                done.set()
+
+    threads = [threading.Thread(target=caller, args=(i,)) for i in range(len(work))]
+    for t in threads:
+        t.start()
+    while not done.wait(0.01):
+        moehip.check(moehip.lib().moe_weight_cache_clear())
+    for t in threads:
+        t.join()
+    assert not wrong, wrong
