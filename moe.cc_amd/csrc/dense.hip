@@ -1753,20 +1753,27 @@ moe_status launch_mfma(const DenseArgs& a, hipStream_t s) {
 // 64 x 64 116, 160, 246, 586 for m = 1, 2, 3, 8; 64 x 80 145, 199, 305 for m =
 // 1, 2, 3.  Small tiles spread few tokens over the CUs, large ones spend less
 // on operands per product.
-template <bool ANY>
-moe_status launch_mfma_best(const DenseArgs& a, hipStream_t s) {
+// A grid holds 65535 row tiles: taller products keep the 64-row shapes (up to
+// 4,194,240 rows); -1 past those.
+int mfma_shape(int M, int N) {
   struct Shape { int rx, rw, step, odd; };
   static const Shape shapes[4] = {{32, 32, 22, 10}, {32, 64, 40, 18}, {64, 64, 75, 42}, {64, 80, 95, 50}};
-  int best = 0;
+  int best = -1;
   double tbest = 0.0;
   for (int i = 0; i < 4; ++i) {
     const Shape& h = shapes[i];
-    const long long blocks = (long long)((a.N + h.rw - 1) / h.rw) * ((a.M + h.rx - 1) / h.rx);
-    const long long m = (blocks + 255) / 256;
+    const long long tiles = ((long long)M + h.rx - 1) / h.rx;
+    if (tiles > 65535) continue;
+    const long long m = (((long long)N + h.rw - 1) / h.rw * tiles + 255) / 256;
     const double t = (double)m * h.step + (m & 1) * h.odd;
-    if (i == 0 || t < tbest) { best = i; tbest = t; }
+    if (best < 0 || t < tbest) { best = i; tbest = t; }
   }
-  switch (best) {
+  return best;
+}
+
+template <bool ANY>
+moe_status launch_mfma_best(const DenseArgs& a, int shape, hipStream_t s) {
+  switch (shape) {
     case 0: return launch_mfma<2, 1, 64, 2, ANY>(a, s);
     case 1: return launch_mfma<2, 2, 32, 2, ANY>(a, s);
     case 2: return launch_mfma<4, 4, 32, 2, ANY>(a, s);
@@ -1905,8 +1912,9 @@ moe_status dense_matmul(const DenseArgs& a, hipStream_t s) {
     if (a.pack_dtype == 3) return launch_gemv<16, true, 3, 1>(a, s);
     return launch_gemv<16, true, 0, 1>(a, s);
   }
-  if (!vec && a.K >= 4 && (a.M + 31) / 32 <= 65535) return launch_mfma_best<true>(a, s);
-  if (!vec) {
+  const int mfma = mfma_shape(a.M, a.N);
+  if (!vec && a.K >= 4 && mfma >= 0) return launch_mfma_best<true>(a, mfma, s);
+  if (!vec || mfma < 0) {
     const long long total = (long long)a.M * a.N;
     hipLaunchKernelGGL(dense_generic_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, a);
     return check_hip(hipGetLastError(), "dense generic launch");
@@ -1963,7 +1971,7 @@ moe_status dense_matmul(const DenseArgs& a, hipStream_t s) {
     // tiles are never slower (16 x 1100 x 1024: 21 against 16)
     return launch_gemv<4, false, 0, 1>(a, s);
   } else {
-    return launch_mfma_best<false>(a, s);
+    return launch_mfma_best<false>(a, mfma, s);
   }
 }
 

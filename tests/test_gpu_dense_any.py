@@ -17,7 +17,8 @@ def bits(a):
 # (M, N, K, floats past a 16-byte boundary of A, of W)
 SHAPES = [(1, 1, 1, 0, 0), (1, 70, 3, 0, 0), (4, 33, 63, 0, 0), (1, 1000, 65, 0, 0), (7, 31, 129, 1, 3),
           (33, 40, 1030, 0, 0), (20, 33, 64, 1, 0), (2, 50, 128, 0, 2), (500, 2050, 31, 0, 0), (505, 5100, 33, 0, 1),
-          (1000, 8150, 35, 0, 0), (1000, 8150, 32, 3, 3)]
+          (1000, 8150, 35, 0, 0), (1000, 8150, 32, 3, 3),
+          (2097185, 2, 5, 0, 0)]
 
 
 @pytest.mark.parametrize("M,N,K,oa,ow", SHAPES)
