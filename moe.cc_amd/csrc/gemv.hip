@@ -293,8 +293,12 @@ __global__ __launch_bounds__(kBlock) void qgemv_fused(TiledArgs a) {
 // quantizes its MT tokens' activations into LDS once (16-byte units per
 // chunk and limb: Q8 the 16 columns, Q4 the 16 even columns, then the 16 odd
 // ones), then L lanes share a row, RPT rows a lane, each unit read from LDS
-// serving RPT rows.  Activations past two limbs take the exact fp32
-// fallback.
+// serving RPT rows.  A block whose activations need more than two limbs (Q8
+// |x| > 258, Q4 |x| > 4681) goes over its rows twice, for the lower and the
+// upper two; the lane that stores an output leaves the lower half of its dot
+// there meanwhile.  (Q8 [8192 x 2046], 5 tokens of |x| about 300: 34 us with a
+// wave a row converting every activation per row, 476 with that inside these
+// blocks, 30 so.)
 //
 // Bound: latency at a few MB (each block: its activations, two or three
 // dependent chunk loads, the reduction).  Q8 [1000 x 1030], 7 tokens: 20.2
@@ -308,15 +312,6 @@ struct AnyArgs {
   QJob one;
   int blocks_per_job;
   int rows_per_block;
-};
-
-struct AnyEpi {
-  const float* S;
-  float* C;
-  float div;
-  __device__ void operator()(int row, const uint32_t (&tot)[1][1]) const {
-    C[row] = qdot_epilogue(tot[0][0], div, S[row]);
-  }
 };
 
 template <bool Q4, int MT, int L, int RPT>
@@ -345,31 +340,37 @@ __global__ __launch_bounds__(kBlock) void qgemv_any(AnyArgs a) {
     if (o < dup) act[((size_t)(u / U) * NC * U + (size_t)(NC - 1) * U + u % U) * 16 + o] = 0;
   }
   __syncthreads();
-  // quantize: column k of byte position p (Q8 k, Q4 k / 2) sits in chunk
-  // p / 16, the last chunk starting at byte rb - 16
+  // quantize (limbs 2H and 2H + 1): column k of byte position p (Q8 k, Q4 k /
+  // 2) sits in chunk p / 16, the last chunk starting at byte rb - 16
   int32_t lo = 0, hi = 0;   // limbs_needed is monotone in |value|
   uint32_t sum[MT];
 #pragma unroll
   for (int t = 0; t < MT; ++t) sum[t] = 0u;
-  for (int k = tid; k < K; k += kBlock) {
-    float x[MT];
+  auto quantize = [&](auto h_tag) {
+    constexpr int H = decltype(h_tag)::value;
+    for (int k = tid; k < K; k += kBlock) {
+      float x[MT];
 #pragma unroll
-    for (int t = 0; t < MT; ++t) x[t] = job.A[(size_t)(m0 + min(t, ntok - 1)) * a.sh.lda + k];
-    const int pos = Q4 ? k / 2 : k;
-    const int c = min(pos / 16, NC - 1), o = c < NC - 1 ? pos % 16 : pos - (rb - 16);
-    uint8_t* d = act + ((size_t)c * U + (Q4 ? k % 2 : 0)) * 16 + o;
+      for (int t = 0; t < MT; ++t) x[t] = job.A[(size_t)(m0 + min(t, ntok - 1)) * a.sh.lda + k];
+      const int pos = Q4 ? k / 2 : k;
+      const int c = min(pos / 16, NC - 1), o = c < NC - 1 ? pos % 16 : pos - (rb - 16);
+      uint8_t* d = act + ((size_t)c * U + (Q4 ? k % 2 : 0)) * 16 + o;
 #pragma unroll
-    for (int t = 0; t < MT; ++t) {
-      const int32_t v = f2i_trunc_x86(x[t] * div);
-      lo = min(lo, v);
-      hi = max(hi, v);
-      uint32_t b[4];
-      split_limbs(v, b);
-      d[(size_t)(2 * t) * NC * U * 16] = (uint8_t)b[0];
-      d[(size_t)(2 * t + 1) * NC * U * 16] = (uint8_t)b[1];
-      sum[t] += (uint32_t)v;
+      for (int t = 0; t < MT; ++t) {
+        const int32_t v = f2i_trunc_x86(x[t] * div);
+        uint32_t b[4];
+        split_limbs(v, b);
+        d[(size_t)(2 * t) * NC * U * 16] = (uint8_t)b[2 * H];
+        d[(size_t)(2 * t + 1) * NC * U * 16] = (uint8_t)b[2 * H + 1];
+        if constexpr (H == 0) {
+          lo = min(lo, v);
+          hi = max(hi, v);
+          sum[t] += (uint32_t)v;
+        }
+      }
     }
-  }
+  };
+  quantize(std::integral_constant<int, 0>());
   const int nl = max(limbs_needed(lo), limbs_needed(hi));
   if (nl > 1) atomicMax(&nl_s, nl);
   if constexpr (Q4) {
@@ -381,34 +382,29 @@ __global__ __launch_bounds__(kBlock) void qgemv_any(AnyArgs a) {
   }
   __syncthreads();
   const int nlb = nl_s;
-  if (nlb > 2) {
-    const uint8_t* W[1] = {job.W};
-    for (int t = 0; t < ntok; ++t) {
-      AnyEpi epi{job.S, job.C + (size_t)(m0 + t) * a.sh.ldc, div};
-      generic_rows_fp32<Q4, 1>(W, a.sh.rs, K, job.A + (size_t)(m0 + t) * a.sh.lda, r0, r1, epi, wave, kWaves);
-    }
-    return;
-  }
-  auto run = [&](auto nl_tag) {
-    constexpr int NL = decltype(nl_tag)::value;
+  // HALF 0: the whole dots; 1: of the lower two limbs of four, left in C as
+  // bits; 2: of the upper two, added to those
+  auto run = [&](auto nl_tag, auto half_tag) {
+    constexpr int NL = decltype(nl_tag)::value, HALF = decltype(half_tag)::value;
+    constexpr int R = HALF ? 1 : RPT;   // (four rows' registers are the usual path's)
     const int sub = lane / L, l = lane % L;
-    for (int rb0 = r0 + (wave * G + sub) * RPT; rb0 - sub * RPT < r1; rb0 += kWaves * G * RPT) {
-      const uint8_t* w[RPT];
+    for (int rb0 = r0 + (wave * G + sub) * R; rb0 - sub * R < r1; rb0 += kWaves * G * R) {
+      const uint8_t* w[R];
 #pragma unroll
-      for (int i = 0; i < RPT; ++i) w[i] = job.W + (size_t)min(rb0 + i, r1 - 1) * (size_t)a.sh.rs;
-      int acc[RPT][MT][NL];
+      for (int i = 0; i < R; ++i) w[i] = job.W + (size_t)min(rb0 + i, r1 - 1) * (size_t)a.sh.rs;
+      int acc[R][MT][NL];
 #pragma unroll
-      for (int i = 0; i < RPT; ++i)
+      for (int i = 0; i < R; ++i)
 #pragma unroll
         for (int t = 0; t < MT; ++t)
 #pragma unroll
           for (int n = 0; n < NL; ++n) acc[i][t][n] = 0;
-      auto load = [&](int c, u32x4 (&v)[RPT]) {
+      auto load = [&](int c, u32x4 (&v)[R]) {
         const int at = min(16 * c, rb - 16);
 #pragma unroll
-        for (int i = 0; i < RPT; ++i) v[i] = *reinterpret_cast<const u32x4_any*>(w[i] + at);
+        for (int i = 0; i < R; ++i) v[i] = *reinterpret_cast<const u32x4_any*>(w[i] + at);
       };
-      u32x4 cur[RPT], nxt[RPT];
+      u32x4 cur[R], nxt[R];
       if (l < NC) load(l, cur);
       for (int c = l; c < NC; c += L) {
         if (c + L < NC) load(c + L, nxt);
@@ -419,40 +415,64 @@ __global__ __launch_bounds__(kBlock) void qgemv_any(AnyArgs a) {
             const u32x4* q = any_lds + ((size_t)(2 * t + n) * NC + c) * U;
             const u32x4 x0 = q[0];
 #pragma unroll
-            for (int i = 0; i < RPT; ++i)
+            for (int i = 0; i < R; ++i)
 #pragma unroll
               for (int d = 0; d < 4; ++d)
                 acc[i][t][n] = dot4(Q4 ? cur[i][d] & 0x0F0F0F0Fu : cur[i][d], x0[d], acc[i][t][n]);
             if constexpr (Q4) {
               const u32x4 x1 = q[1];
 #pragma unroll
-              for (int i = 0; i < RPT; ++i)
+              for (int i = 0; i < R; ++i)
 #pragma unroll
                 for (int d = 0; d < 4; ++d)
                   acc[i][t][n] = dot4((cur[i][d] >> 4) & 0x0F0F0F0Fu, x1[d], acc[i][t][n]);
             }
           }
 #pragma unroll
-        for (int i = 0; i < RPT; ++i) cur[i] = nxt[i];
+        for (int i = 0; i < R; ++i) cur[i] = nxt[i];
       }
+      // lane j of the row group finishes output j (row j / MT, token j % MT)
+      // and j + L: one lane finishing all of them would do RPT MT divisions
+      // one after another
+      constexpr int NO = (R * MT + L - 1) / L;
+      uint32_t v[NO];
 #pragma unroll
-      for (int i = 0; i < RPT; ++i) {
-        const int row = rb0 + i;
-        const float sc = job.S[min(row, r1 - 1)];
+      for (int i = 0; i < R; ++i)
 #pragma unroll
         for (int t = 0; t < MT; ++t) {
-          uint32_t v = (uint32_t)acc[i][t][0];
-          if constexpr (NL == 2) v += (uint32_t)acc[i][t][1] << 8;
-          v = group_sum_dpp<L>(v);
-          if constexpr (Q4) v -= 8u * asum[t];
-          if (l == 0 && t < ntok && row < r1)
-            job.C[(size_t)(m0 + t) * a.sh.ldc + row] = qdot_epilogue(v, div, sc);
+          uint32_t d = (uint32_t)acc[i][t][0];
+          if constexpr (NL == 2) d += (uint32_t)acc[i][t][1] << 8;
+          d = group_sum_dpp<L>(d);
+          const int j = i * MT + t;
+          v[j / L] = j % L == 0 || l == j % L ? d : v[j / L];
+        }
+#pragma unroll
+      for (int u = 0; u < NO; ++u) {
+        const int j = u * L + l, t = j % MT, row = rb0 + j / MT;
+        if (j >= R * MT || t >= ntok || row >= r1) continue;
+        float* out = job.C + (size_t)(m0 + t) * a.sh.ldc + row;
+        if constexpr (HALF == 1) {
+          *out = __builtin_bit_cast(float, v[u]);
+        } else {
+          if constexpr (HALF == 2) v[u] = (v[u] << 16) + __builtin_bit_cast(uint32_t, *out);
+          if constexpr (Q4) v[u] -= 8u * asum[t];
+          *out = qdot_epilogue(v[u], div, job.S[row]);
         }
       }
     }
   };
-  if (nlb == 1) run(std::integral_constant<int, 1>());
-  else run(std::integral_constant<int, 2>());
+  using std::integral_constant;
+  if (nlb == 1) {
+    run(integral_constant<int, 1>(), integral_constant<int, 0>());
+  } else if (nlb == 2) {
+    run(integral_constant<int, 2>(), integral_constant<int, 0>());
+  } else {
+    run(integral_constant<int, 2>(), integral_constant<int, 1>());
+    __syncthreads();   // every wave is done with the lower limbs
+    quantize(integral_constant<int, 1>());
+    __syncthreads();
+    run(integral_constant<int, 2>(), integral_constant<int, 2>());
+  }
 }
 
 template <bool Q4>

@@ -253,9 +253,8 @@ __device__ __forceinline__ uint32_t dpp_u32(uint32_t v) {
   return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xF, 0xF, true);
 }
 
-// Sum over groups of W consecutive lanes (W = 4, 8, 16, 32, 64).  For W <= 16
-// every lane of the group gets the total; for W = 32 / 64 lane 0 of the group
-// is guaranteed to have it.
+// Sum over groups of W consecutive lanes (W = 4, 8, 16, 32, 64); every lane of
+// the group gets the total.
 template <int W>
 __device__ __forceinline__ uint32_t group_sum_dpp(uint32_t v) {
   v += dpp_u32<0xB1>(v);                 // quad_perm [1,0,3,2]

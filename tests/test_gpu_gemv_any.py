@@ -25,7 +25,7 @@ SHAPES = [(2, 5, 16), (2, 7, 17), (2, 9, 48), (2, 33, 31), (2, 20, 496), (2, 20,
 
 
 @pytest.mark.parametrize("dtype,N,K", SHAPES)
-@pytest.mark.parametrize("M,scale", [(1, 1.0), (4, 0.05), (5, 30.0), (9, 1.0), (2, 1e5)])
+@pytest.mark.parametrize("M,scale", [(1, 1.0), (4, 0.05), (5, 30.0), (9, 1.0), (2, 1e5), (9, 1e5), (1, 1e9)])
 def test_gemv_any_shapes(moehip, dtype, N, K, M, scale):
     print("gemv any case", dtype, N, K, M, scale, flush=True)
     assert moehip.gemv_variant(dtype, M, N, K) == "generic"
