@@ -298,7 +298,7 @@ __global__ __launch_bounds__(kBlock) void qgemv_fused(TiledArgs a) {
 // upper two; the lane that stores an output leaves the lower half of its dot
 // there meanwhile.  (Q8 [8192 x 2046], 5 tokens of |x| about 300: 34 us with a
 // wave a row converting every activation per row, 476 with that inside these
-// blocks, 30 so.)
+// blocks, 25 so.)
 //
 // Bound: latency at a few MB (each block: its activations, two or three
 // dependent chunk loads, the reduction).  Q8 [1000 x 1030], 7 tokens: 20.2
@@ -741,10 +741,18 @@ bool qgemv_tiled_ok(const QShape& sh, const void* w_base) {
 
 // qgemv_any where its tables fit (false: the caller runs qgemv_generic):
 // even Q4 columns, rows of at least one chunk, two limbs of MT tokens within
-// 129 KB of LDS.  MT: 1, 4 or 8 tokens a block.  A whole wave per row while the rows
-// are few (the launch is latency-bound then), 16 lanes per row where a row
-// has under 32 chunks; with several tokens and 4096 rows or more, 16 lanes
-// and four rows each, so that one LDS read serves four rows.
+// 129 KB of LDS.  MT: 1, 4 or 8 tokens a block.
+//
+// Lanes a row: with `rows` = rows x token groups, 16 lanes where a row has
+// under 32 chunks or there are rows enough to fill the chip that way, else a
+// wave.  Measured, us, wave / 16 lanes: Q8 K = 1030 and 5000, one token, 1000
+// rows 4.9 / 5.2 and 8.0 / 10.3, 4099 rows 6.5 / 5.3 and 11.5 / 13.1, 8192
+// rows 8.9 / 5.6 and 17.6 / 17.6; K = 3000, 4 tokens 2050 rows 9.6 / 10.6,
+// 4099 rows 13.0 / 11.1, 16 tokens 2050 rows 24 / 18.  Four rows a lane, so
+// that one LDS read serves four, only where the rows and their chunks are
+// many, one token group less often than several (one row a lane / four): K =
+// 250, 5 tokens 4099 rows 5.7 / 7.5, 64 tokens 13.5 / 11.5; K = 3000, 8192
+// rows, 8 tokens 20 / 25, 16 tokens 36 / 25, 64 tokens 108 / 53.
 bool launch_any(const QShape& sh, const QJob* jobs_dev, const QJob& one, int njobs, hipStream_t stream,
                 hipError_t* err) {
   const bool q4 = sh.dtype == 3;
@@ -752,17 +760,19 @@ bool launch_any(const QShape& sh, const QJob* jobs_dev, const QJob& one, int njo
   if ((q4 && (sh.K & 1)) || rb < 16 || sh.K > 65536 || sh.rs != rb) return false;
   int mt = sh.M == 1 ? 1 : sh.M <= 4 ? 4 : 8;
   while (mt > 1 && (long long)mt * sh.K > 65536) mt = mt == 8 ? 4 : 1;
-  const int nc = (int)((rb + 15) / 16);
-  const bool wide = mt > 1 && sh.N >= 4096;
-  const int L = wide || nc < 32 ? 16 : 64, rpt = wide ? 4 : 1;
+  const int nc = (int)((rb + 15) / 16), nu = q4 ? 2 * nc : nc;
+  const long long gy = ((long long)sh.M + mt - 1) / mt, rows = (long long)sh.N * njobs * gy;
+  const bool wide = mt > 1 && sh.N >= 4096 && (rows >= 32768 || rows * nu >= (gy > 1 ? 1 << 20 : 1 << 21));
+  const bool many = mt > 1 ? rows >= std::max(2048, 12 * nc) : rows >= std::max(4096, 20 * nc);
+  const int L = wide || many || nc < 32 ? 16 : 64, rpt = wide ? 4 : 1;
   const int unit = kWaves * (kWave / L) * rpt;
   const long long units = ((long long)sh.N + unit - 1) / unit;
   const long long per = std::max<long long>(1, (units * njobs + 2047) / 2048);   // at most ~2048 blocks a token group
   AnyArgs a{sh, jobs_dev, one, (int)((units + per - 1) / per), (int)std::min<long long>(per * unit, INT_MAX / 2)};
-  const long long gx = (long long)a.blocks_per_job * njobs, gy = (sh.M + mt - 1) / mt;
+  const long long gx = (long long)a.blocks_per_job * njobs;
   if (gx > INT_MAX || gy > 65535) return false;
   *err = hipSuccess;
-  const size_t lds = (size_t)mt * 2 * nc * (q4 ? 2 : 1) * 16;
+  const size_t lds = (size_t)mt * 2 * nu * 16;
   const dim3 grid((unsigned)gx, (unsigned)gy);
   auto go = [&](auto q4_tag, auto mt_tag, auto l_tag, auto r_tag) {
     auto* fn = qgemv_any<decltype(q4_tag)::value, decltype(mt_tag)::value, decltype(l_tag)::value,
@@ -775,8 +785,9 @@ bool launch_any(const QShape& sh, const QJob* jobs_dev, const QJob& one, int njo
   };
   using std::integral_constant;
   auto with_mt = [&](auto q4_tag, auto mt_tag) {
-    if (wide) go(q4_tag, mt_tag, integral_constant<int, 16>(), integral_constant<int, 4>());
-    else if (L == 16) go(q4_tag, mt_tag, integral_constant<int, 16>(), integral_constant<int, 1>());
+    if constexpr (decltype(mt_tag)::value > 1)
+      if (wide) return go(q4_tag, mt_tag, integral_constant<int, 16>(), integral_constant<int, 4>());
+    if (L == 16) go(q4_tag, mt_tag, integral_constant<int, 16>(), integral_constant<int, 1>());
     else go(q4_tag, mt_tag, integral_constant<int, 64>(), integral_constant<int, 1>());
   };
   auto with_q = [&](auto q4_tag) {

@@ -14,18 +14,19 @@ def bits(a):
 
 # (dtype, N, K): rows of exactly one chunk, one byte more, whole chunks, a
 # last chunk that repeats 15 bytes; 31 / 32 / 33 chunks (16 lanes a row below
-# 32, a wave from 32), 64 and 65 chunks (one and two per lane); 4096 rows and
-# more with several tokens (four rows a lane); the largest K of each token
-# count (8 x 8192, 4 x 16384, 1 x 65536) and one past
+# 32, a wave from 32), 64 and 65 chunks (one and two per lane); 2048 rows and
+# more with several tokens, 4096 with one (16 lanes a row for longer rows too),
+# 4096 rows and more with 70 tokens (four rows a lane); the largest K of each
+# token count (8 x 8192, 4 x 16384, 1 x 65536) and one past
 SHAPES = [(2, 5, 16), (2, 7, 17), (2, 9, 48), (2, 33, 31), (2, 20, 496), (2, 20, 511), (2, 17, 513),
           (2, 130, 1023), (2, 130, 1030), (2, 4099, 66), (2, 9, 8191), (2, 9, 8193), (2, 6, 16385),
-          (2, 3, 65535), (2, 3, 65537),
+          (2, 3, 65535), (2, 3, 65537), (2, 2060, 1030), (2, 4100, 1023),
           (3, 5, 32), (3, 7, 34), (3, 33, 62), (3, 20, 992), (3, 17, 1026), (3, 130, 2050),
-          (3, 4097, 70), (3, 9, 8190), (3, 9, 8194), (3, 6, 16386), (3, 3, 65534)]
+          (3, 4097, 70), (3, 9, 8190), (3, 9, 8194), (3, 6, 16386), (3, 3, 65534), (3, 2051, 1090)]
 
 
 @pytest.mark.parametrize("dtype,N,K", SHAPES)
-@pytest.mark.parametrize("M,scale", [(1, 1.0), (4, 0.05), (5, 30.0), (9, 1.0), (2, 1e5), (9, 1e5), (1, 1e9)])
+@pytest.mark.parametrize("M,scale", [(1, 1.0), (4, 0.05), (5, 30.0), (9, 1.0), (2, 1e5), (9, 1e5), (1, 1e9), (70, 300.0)])
 def test_gemv_any_shapes(moehip, dtype, N, K, M, scale):
     print("gemv any case", dtype, N, K, M, scale, flush=True)
     assert moehip.gemv_variant(dtype, M, N, K) == "generic"
