@@ -13,8 +13,10 @@
 //      stream rows with double-buffered dwordx4 loads (LPR lanes per row, a
 //      row = LPR*P*16 bytes), dot on v_dot4_i32_i8 and reduce across the
 //      row's lanes with DPP.  No LDS, no block barriers in the main loop.
-// Shapes without a tiled geometry (row bytes not LPR*P*16, unaligned rows,
-// odd-K Q4) and Q4 activations that need 4 limbs use a one-wave-per-row
+// Shapes without a tiled geometry (other row bytes, unaligned rows) run
+// qgemv_any: one launch, activations quantized per block, unaligned row chunks.
+// What that does not take either (odd-K Q4, rows under 16 bytes, K past 65536)
+// and Q4 activations of a tiled shape that need 4 limbs use a one-wave-per-row
 // kernel with plain int32 arithmetic on the fp32 activations.
 #include <algorithm>
 #include <climits>
@@ -629,12 +631,6 @@ void release_gemv_workspace() {
   g_ws_bytes = 0;
 }
 
-const char* qgemv_variant_name(const QShape& sh, const void* w_base) {
-  Variant v;
-  if (select_tiled(sh, w_base, &v)) return v.name;
-  return "generic";
-}
-
 hipError_t launch_act_pack(const QShape& sh, const QJob* jobs_dev, const QJob& one, int njobs,
                            uint8_t* tabs, hipStream_t stream) {
   const size_t tb = act_table_bytes(sh.K);
@@ -739,7 +735,9 @@ bool qgemv_tiled_ok(const QShape& sh, const void* w_base) {
   return select_tiled(sh, w_base, &v);
 }
 
-// qgemv_any where its tables fit (false: the caller runs qgemv_generic):
+namespace {
+
+// The shape of a qgemv_any launch, where its tables fit (else qgemv_generic):
 // even Q4 columns, rows of at least one chunk, two limbs of MT tokens within
 // 129 KB of LDS.  MT: 1, 4 or 8 tokens a block.
 //
@@ -753,8 +751,14 @@ bool qgemv_tiled_ok(const QShape& sh, const void* w_base) {
 // many, one token group less often than several (one row a lane / four): K =
 // 250, 5 tokens 4099 rows 5.7 / 7.5, 64 tokens 13.5 / 11.5; K = 3000, 8192
 // rows, 8 tokens 20 / 25, 16 tokens 36 / 25, 64 tokens 108 / 53.
-bool launch_any(const QShape& sh, const QJob* jobs_dev, const QJob& one, int njobs, hipStream_t stream,
-                hipError_t* err) {
+struct AnyPlan {
+  int mt, L, rpt;   // tokens a block, lanes a row, rows a lane
+  int blocks_per_job, rows_per_block;
+  long long gx, gy;
+  size_t lds;
+};
+
+bool plan_any(const QShape& sh, int njobs, AnyPlan* p) {
   const bool q4 = sh.dtype == 3;
   const long long rb = q4 ? sh.K / 2 : sh.K;
   if ((q4 && (sh.K & 1)) || rb < 16 || sh.K > 65536 || sh.rs != rb) return false;
@@ -764,40 +768,56 @@ bool launch_any(const QShape& sh, const QJob* jobs_dev, const QJob& one, int njo
   const long long gy = ((long long)sh.M + mt - 1) / mt, rows = (long long)sh.N * njobs * gy;
   const bool wide = mt > 1 && sh.N >= 4096 && (rows >= 32768 || rows * nu >= (gy > 1 ? 1 << 20 : 1 << 21));
   const bool many = mt > 1 ? rows >= std::max(2048, 12 * nc) : rows >= std::max(4096, 20 * nc);
-  const int L = wide || many || nc < 32 ? 16 : 64, rpt = wide ? 4 : 1;
-  const int unit = kWaves * (kWave / L) * rpt;
+  p->mt = mt;
+  p->L = wide || many || nc < 32 ? 16 : 64;
+  p->rpt = wide ? 4 : 1;
+  const int unit = kWaves * (kWave / p->L) * p->rpt;
   const long long units = ((long long)sh.N + unit - 1) / unit;
   const long long per = std::max<long long>(1, (units * njobs + 2047) / 2048);   // at most ~2048 blocks a token group
-  AnyArgs a{sh, jobs_dev, one, (int)((units + per - 1) / per), (int)std::min<long long>(per * unit, INT_MAX / 2)};
-  const long long gx = (long long)a.blocks_per_job * njobs;
-  if (gx > INT_MAX || gy > 65535) return false;
-  *err = hipSuccess;
-  const size_t lds = (size_t)mt * 2 * nu * 16;
-  const dim3 grid((unsigned)gx, (unsigned)gy);
-  auto go = [&](auto q4_tag, auto mt_tag, auto l_tag, auto r_tag) {
-    auto* fn = qgemv_any<decltype(q4_tag)::value, decltype(mt_tag)::value, decltype(l_tag)::value,
-                         decltype(r_tag)::value>;
-    if (lds > 60 * 1024)
-      *err = hipFuncSetAttribute((const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if (*err != hipSuccess) return;
-    hipLaunchKernelGGL(fn, grid, dim3(kBlock), lds, stream, a);
-    *err = hipGetLastError();
-  };
-  using std::integral_constant;
-  auto with_mt = [&](auto q4_tag, auto mt_tag) {
-    if constexpr (decltype(mt_tag)::value > 1)
-      if (wide) return go(q4_tag, mt_tag, integral_constant<int, 16>(), integral_constant<int, 4>());
-    if (L == 16) go(q4_tag, mt_tag, integral_constant<int, 16>(), integral_constant<int, 1>());
-    else go(q4_tag, mt_tag, integral_constant<int, 64>(), integral_constant<int, 1>());
-  };
-  auto with_q = [&](auto q4_tag) {
-    if (mt == 8) with_mt(q4_tag, integral_constant<int, 8>());
-    else if (mt == 4) with_mt(q4_tag, integral_constant<int, 4>());
-    else with_mt(q4_tag, integral_constant<int, 1>());
-  };
-  if (q4) with_q(std::true_type());
-  else with_q(std::false_type());
-  return true;
+  p->blocks_per_job = (int)((units + per - 1) / per);
+  p->rows_per_block = (int)std::min<long long>(per * unit, INT_MAX / 2);
+  p->gx = (long long)p->blocks_per_job * njobs;
+  p->gy = gy;
+  p->lds = (size_t)mt * 2 * nu * 16;
+  return p->gx <= INT_MAX && gy <= 65535;
+}
+
+template <bool Q4, int MT, int L, int RPT>
+hipError_t launch_any_variant(const AnyPlan& p, const AnyArgs& a, hipStream_t stream) {
+  static size_t allowed = 60 * 1024;   // dynamic LDS granted so far
+  if (p.lds > allowed) {
+    hipError_t e = hipFuncSetAttribute((const void*)qgemv_any<Q4, MT, L, RPT>,
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)p.lds);
+    if (e != hipSuccess) return e;
+    allowed = p.lds;
+  }
+  hipLaunchKernelGGL((qgemv_any<Q4, MT, L, RPT>), dim3((unsigned)p.gx, (unsigned)p.gy), dim3(kBlock), p.lds, stream, a);
+  return hipGetLastError();
+}
+
+template <bool Q4, int MT>
+hipError_t launch_any_tokens(const AnyPlan& p, const AnyArgs& a, hipStream_t stream) {
+  if constexpr (MT > 1)
+    if (p.rpt == 4) return launch_any_variant<Q4, MT, 16, 4>(p, a, stream);
+  if (p.L == 16) return launch_any_variant<Q4, MT, 16, 1>(p, a, stream);
+  return launch_any_variant<Q4, MT, 64, 1>(p, a, stream);
+}
+
+template <bool Q4>
+hipError_t launch_any(const AnyPlan& p, const AnyArgs& a, hipStream_t stream) {
+  if (p.mt == 8) return launch_any_tokens<Q4, 8>(p, a, stream);
+  if (p.mt == 4) return launch_any_tokens<Q4, 4>(p, a, stream);
+  return launch_any_tokens<Q4, 1>(p, a, stream);
+}
+
+}  // namespace
+
+const char* qgemv_variant_name(const QShape& sh, const void* w_base) {
+  Variant v;
+  if (select_tiled(sh, w_base, &v)) return v.name;
+  AnyPlan p;
+  if (plan_any(sh, 1, &p)) return p.rpt == 4 ? "any_l16r4" : p.L == 16 ? "any_l16" : "any_l64";
+  return "generic";
 }
 
 hipError_t launch_qgemv(const QShape& sh, const QJob* jobs_dev, const QJob& one, int njobs,
@@ -821,8 +841,11 @@ hipError_t launch_qgemv(const QShape& sh, const QJob* jobs_dev, const QJob& one,
     if (e != hipSuccess) return e;
     return launch_qgemv_tables(sh, jobs_dev, one, njobs, g_ws, 0, stream);
   }
-  hipError_t err;
-  if (launch_any(sh, jobs_dev, one, njobs, stream, &err)) return err;
+  AnyPlan p;
+  if (plan_any(sh, njobs, &p)) {
+    const AnyArgs a{sh, jobs_dev, one, p.blocks_per_job, p.rows_per_block};
+    return sh.dtype == 3 ? launch_any<true>(p, a, stream) : launch_any<false>(p, a, stream);
+  }
   const int bpj = (sh.N + kWaves - 1) / kWaves;
   dim3 grid((unsigned)((long long)bpj * njobs), (unsigned)((sh.M + 15) / 16));
   if (sh.dtype == 3)

@@ -1,5 +1,7 @@
 """The untiled-shape GEMV kernel (unaligned 16-byte row chunks, activations
 quantized per block) against the oracle, bit for bit."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -25,11 +27,32 @@ SHAPES = [(2, 5, 16), (2, 7, 17), (2, 9, 48), (2, 33, 31), (2, 20, 496), (2, 20,
           (3, 4097, 70), (3, 9, 8190), (3, 9, 8194), (3, 6, 16386), (3, 3, 65534), (3, 2051, 1090)]
 
 
+def variant(dtype, M, N, K):
+    """The kernel these shapes are meant to reach."""
+    nc = -(-(K if dtype == 2 else K // 2) // 16)
+    if K > 65536:
+        return "generic"
+    mt = next(m for m in (1, 4, 8) if M <= m or m == 8)
+    while mt > 1 and mt * K > 65536:
+        mt = 4 if mt == 8 else 1
+    rows = N * -(-M // mt)
+    if mt > 1 and N >= 4096 and rows >= 32768:
+        return "any_l16r4"
+    many = rows >= max(2048, 12 * nc) if mt > 1 else rows >= max(4096, 20 * nc)
+    return "any_l16" if nc < 32 or many else "any_l64"
+
+
+def test_variants_reached():
+    reached = {variant(d, M, N, K) for d, N, K in SHAPES for M in (1, 5, 70)}
+    assert reached == {"any_l16", "any_l16r4", "any_l64", "generic"}
+    assert any(variant(d, M, N, K) == "any_l16" and K > 1024 for d, N, K in SHAPES for M in (1, 5))
+
+
 @pytest.mark.parametrize("dtype,N,K", SHAPES)
 @pytest.mark.parametrize("M,scale", [(1, 1.0), (4, 0.05), (5, 30.0), (9, 1.0), (2, 1e5), (9, 1e5), (1, 1e9), (70, 300.0)])
 def test_gemv_any_shapes(moehip, dtype, N, K, M, scale):
     print("gemv any case", dtype, N, K, M, scale, flush=True)
-    assert moehip.gemv_variant(dtype, M, N, K) == "generic"
+    assert moehip.gemv_variant(dtype, M, N, K) == variant(dtype, M, N, K)
     seed = dtype * 100000 + N * 31 + K * 7 + M
     A = O.normal(M * K, seed, 0.0, scale).reshape(M, K)
     rb = K if dtype == 2 else K // 2
@@ -46,3 +69,32 @@ def test_gemv_any_shapes(moehip, dtype, N, K, M, scale):
     f = L.moe_matmul_q8_dev if dtype == 2 else L.moe_matmul_q4_dev
     moehip.check(f(dA.ptr, dq.ptr + 33, ds.ptr, dC.ptr, M, N, K), "gemv")
     np.testing.assert_array_equal(bits(dC.download((M, N), np.float32)), bits(want))
+
+
+# (dtype, jobs, M, N, K): rows a multiple of 16 bytes without a tiled
+# geometry; blocks of one row unit and, past 2048 units, of several with a
+# partial last one; 16 lanes and (7 rows) a wave a row; tokens past a block's
+@pytest.mark.parametrize("dtype,nj,M,N,K", [(2, 3, 1, 7, 1040), (2, 5, 4, 100, 96), (3, 5, 9, 100, 96),
+                                            (2, 300, 1, 200, 112), (3, 40, 5, 1000, 96), (2, 2, 2, 9000, 80),
+                                            (3, 9, 3, 4100, 160), (2, 1, 1, 40000, 48)])
+@pytest.mark.parametrize("scale", [1.0, 1e5])
+def test_gemv_any_batched(moehip, dtype, nj, M, N, K, scale):
+    print("gemv any batched", dtype, nj, M, N, K, scale, flush=True)
+    assert moehip.gemv_variant(dtype, M, N, K).startswith("any")
+    rb = K if dtype == 2 else K // 2
+    q = (O.uniform_u32(nj * N * rb, 11 + K) & 0xFF).astype(np.uint8)
+    q = (q.view(np.int8) if dtype == 2 else q).reshape(nj, N, rb)
+    s = O.normal(nj * N, 12, 0.0, 0.01).reshape(nj, N)
+    A = O.normal(nj * M * K, 13 + M, 0.0, scale).reshape(nj, M, K)
+    dq, ds, dA = (moehip.DeviceBuffer.from_array(v) for v in (q, s, A))
+    dC = moehip.DeviceBuffer(nj * M * N * 4)
+    jobs = (moehip.QJob * nj)(*[moehip.QJob(dq.ptr + j * N * rb, ds.ptr + j * N * 4, dA.ptr + j * M * K * 4,
+                                            dC.ptr + j * M * N * 4) for j in range(nj)])
+    dj = moehip.DeviceBuffer(ctypes.sizeof(jobs))
+    L = moehip.lib()
+    moehip.check(L.moe_memcpy_h2d(dj.ptr, ctypes.addressof(jobs), ctypes.sizeof(jobs)))
+    moehip.check(L.moe_matmul_q_batched_dev(dtype, dj.ptr, nj, M, N, K), "batched")
+    got = dC.download((nj, M, N), np.float32)
+    f = O.gemv_q8 if dtype == 2 else O.gemv_q4
+    for j in range(nj):
+        np.testing.assert_array_equal(bits(got[j]), bits(f(A[j], q[j], s[j], N, K)), err_msg=f"job {j}")
