@@ -1755,7 +1755,8 @@ moe_status launch_mfma(const DenseArgs& a, hipStream_t s) {
 // on operands per product.
 // A grid holds 65535 row tiles: taller products keep the 64-row shapes (up to
 // 4,194,240 rows); -1 past those.
-int mfma_shape(int M, int N) {
+// *t: the estimate, clocks per column.
+int mfma_shape(int M, int N, double* t_out) {
   struct Shape { int rx, rw, step, odd; };
   static const Shape shapes[4] = {{32, 32, 22, 10}, {32, 64, 40, 18}, {64, 64, 75, 42}, {64, 80, 95, 50}};
   int best = -1;
@@ -1768,7 +1769,21 @@ int mfma_shape(int M, int N) {
     const double t = (double)m * h.step + (m & 1) * h.odd;
     if (best < 0 || t < tbest) { best = i; tbest = t; }
   }
+  *t_out = tbest;
   return best;
+}
+
+// 5-16 tokens: whether the chain kernel (launch_gemv<4>) takes less time than
+// the tiles.  Its blocks of four rows run per CU as their LDS allows and take
+// about 4 + M clocks a column (M chains side by side), 8% more for each
+// neighbour, and 7200 around that; the tiles 6000 around theirs.  Measured /
+// estimated us, chain and tiles: 9 x 2048 x 2048 14 / 15 and 30 / 30; 8 x 5120 x
+// 2048 36 / 41 and 31 / 30; 12 x 64 x 8192 56 / 58 and 111 / 112; 16 x 2048 x
+// 1024 22 / 23 and 16 / 16; 12 x 2048 x 64 8 / 7 and 3 / 3.
+bool chain_beats_mfma(int M, int N, int K, double t_mfma) {
+  const int per_cu = M <= 6 ? 3 : M <= 9 ? 2 : 1;
+  const long long rounds = (((long long)N + 3) / 4 + 256 * per_cu - 1) / (256 * per_cu);
+  return (double)rounds * (K * (4.0 + M) * (0.92 + 0.08 * per_cu) + 7200.0) <= K * t_mfma + 6000.0;
 }
 
 template <bool ANY>
@@ -1912,7 +1927,8 @@ moe_status dense_matmul(const DenseArgs& a, hipStream_t s) {
     if (a.pack_dtype == 3) return launch_gemv<16, true, 3, 1>(a, s);
     return launch_gemv<16, true, 0, 1>(a, s);
   }
-  const int mfma = mfma_shape(a.M, a.N);
+  double t_mfma = 0.0;
+  const int mfma = mfma_shape(a.M, a.N, &t_mfma);
   if (!vec && a.K >= 4 && mfma >= 0) return launch_mfma_best<true>(a, mfma, s);
   if (!vec || mfma < 0) {
     const long long total = (long long)a.M * a.N;
@@ -1964,11 +1980,7 @@ moe_status dense_matmul(const DenseArgs& a, hipStream_t s) {
     return launch_gemv<8, false, 0, kNpOne, 1>(a, s);
   } else if (a.M <= 4) {
     return launch_gemv<16, false, 0, 1>(a, s);
-  } else if (a.M <= 8 && (long long)a.M * a.N < 40000) {
-    // the chain kernel costs ~6 us per 1024 rows at M = 8, K = 2048, the MFMA
-    // tiles 30 us up to 8192 rows: 22 against 30 us at 5 x 5120, 35 against
-    // 30 at 8 x 5120, 23 against 57 at 8 x 2048 x 4096; from 9 tokens the
-    // tiles are never slower (16 x 1100 x 1024: 21 against 16)
+  } else if (a.M <= 16 && chain_beats_mfma(a.M, a.N, a.K, t_mfma)) {
     return launch_gemv<4, false, 0, 1>(a, s);
   } else {
     return launch_mfma_best<false>(a, mfma, s);

@@ -26,12 +26,15 @@ def f32_dev(moehip, A, W):
 
 # (M, N, K): one chunk and less, chunk tails of 4..60 columns, one row, rows
 # and tokens one past a tile; the 32 x 64, 64 x 64 and 64 x 80 tiles with
-# partial last tiles (many blocks, few columns); 9-16 tokens past 1024 rows
-# and 5 tokens past 8000 (below, the chain kernel); more 32-row, then 64-row
-# tiles than a grid holds
+# partial last tiles (many blocks, few columns); 5-16 tokens on both sides of
+# the chain kernel's rule (its third, second and only block a CU: 6, 9 and 10
+# tokens; one row past a round of its blocks); more 32-row, then 64-row tiles
+# than a grid holds
 SHAPES = [(17, 1, 4), (17, 31, 32), (32, 32, 60), (33, 33, 64), (31, 79, 68), (65, 81, 100),
           (48, 130, 2044), (500, 2050, 36), (505, 5100, 68), (1000, 8150, 36), (9, 1025, 2048),
           (16, 1100, 68), (5, 8001, 132), (5, 7999, 132), (8, 4999, 64), (8, 5001, 64),
+          (9, 2048, 2048), (9, 2049, 2048), (10, 1024, 4100), (10, 1025, 4100), (6, 3072, 516), (6, 3073, 516),
+          (7, 257, 8192), (16, 64, 8192), (12, 1030, 8192),
           (2097185, 3, 4), (4194305, 3, 4)]
 
 
