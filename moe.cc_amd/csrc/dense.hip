@@ -790,8 +790,8 @@ __global__ __launch_bounds__(256, ANY && NB >= 4 ? 3 : 4) void dense_mfma_kernel
     }
 }
 
-// Any shape or alignment: one thread per output, plain loads (rows under
-// four columns, more rows than a grid of tiles takes).
+// Any shape or alignment: one thread per output, plain loads (unaligned rows
+// of a few columns, more rows than a grid of tiles takes).
 __global__ __launch_bounds__(256) void dense_generic_kernel(DenseArgs a) {
   const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
   if (i >= (long long)a.M * a.N) return;
@@ -1929,7 +1929,13 @@ moe_status dense_matmul(const DenseArgs& a, hipStream_t s) {
   }
   double t_mfma = 0.0;
   const int mfma = mfma_shape(a.M, a.N, &t_mfma);
-  if (!vec && a.K >= 4 && mfma >= 0) return launch_mfma_best<true>(a, mfma, s);
+  // unaligned: the tiles, but a thread an output for a few short rows (thread /
+  // tiles: 16 x 1000 x 7 2.9 / 4.0 us, 300 x 2048 x 5 4.4 / 6.0, 300 x 5120 x 5 7.4 /
+  // 6.5, 300 x 256 x 13 3.7 / 4.1, 32 x 5120 x 13 4.9 / 4.2, 16 x 1000 x 21 3.7 / 4.0,
+  // 33 x 2048 x 21 4.9 / 4.1)
+  const long long thread_work = a.K < 8 ? 4 << 20 : a.K < 16 ? 3 << 19 : a.K < 24 ? 1 << 20 : 0;
+  const bool few_products = (long long)a.M * a.N <= thread_work / a.K;
+  if (!vec && a.K >= 4 && mfma >= 0 && !few_products) return launch_mfma_best<true>(a, mfma, s);
   if (!vec || mfma < 0) {
     const long long total = (long long)a.M * a.N;
     hipLaunchKernelGGL(dense_generic_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, a);

@@ -1,6 +1,6 @@
 """The fp32 product on rows of any length and 4-byte alignment against the
 oracle's sequential loop, bit for bit: lengths under, at and past a chunk of
-its four tile shapes, every remainder of four columns, one row and one token,
+its four tile shapes, few short rows (a thread an output), every remainder of four columns, one row and one token,
 and aligned lengths read from unaligned addresses."""
 import numpy as np
 import pytest
@@ -18,7 +18,8 @@ def bits(a):
 SHAPES = [(1, 1, 1, 0, 0), (1, 70, 3, 0, 0), (4, 33, 63, 0, 0), (1, 1000, 65, 0, 0), (7, 31, 129, 1, 3),
           (33, 40, 1030, 0, 0), (20, 33, 64, 1, 0), (2, 50, 128, 0, 2), (500, 2050, 31, 0, 0), (505, 5100, 33, 0, 1),
           (1000, 8150, 35, 0, 0), (1000, 8150, 32, 3, 3),
-          (2097185, 2, 5, 0, 0)]
+          (2097185, 2, 5, 0, 0), (4, 33, 7, 0, 0), (300, 2048, 5, 0, 0), (300, 2800, 5, 0, 0), (64, 2000, 9, 0, 0),
+          (20, 300, 15, 1, 1), (20, 300, 17, 0, 0), (5, 1000, 23, 0, 0), (5, 1000, 25, 0, 0), (9, 50, 8, 1, 0)]
 
 
 @pytest.mark.parametrize("M,N,K,oa,ow", SHAPES)
