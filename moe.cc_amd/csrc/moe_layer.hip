@@ -544,34 +544,37 @@ __global__ __launch_bounds__(kTileBlock) void gate_up_down_kernel(FuseArgs f) {
 
 // rmsnorm (test_model_trace.c:241-255): one block per token; the squares
 // x_i * x_i are formed by all threads into LDS and summed in order by
-// block_seq_sum (msq / D, 1 / sqrtf(msq + eps)).  Latency: 512 threads give
-// each candidate chain of the sum a thread of its own, and a row of up to 2048
-// columns is read once (5 tokens 7.5 -> 4.6 us, 512 tokens 8.7 -> 6.6).
-constexpr int kRmsThreads = 512;
+// block_seq_sum (msq / D, 1 / sqrtf(msq + eps)).  Few rows are latency: 512
+// threads give each candidate chain of the sum a thread of its own and read
+// the first 2048 columns once (2048 columns, 5 tokens 5.8 -> 4.5 us with 256,
+// 512 tokens 6.9 -> 6.4).  Two such blocks fit a CU: past 512 rows they take a
+// second round, and 256 threads a row are better (2048 rows of 2048 columns
+// 19.2 -> 14.1, of 64 10.6 -> 5.7, of 1001 145 -> 69).
 typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
 
-__global__ __launch_bounds__(kRmsThreads) void rmsnorm_kernel(const float* __restrict__ x,
-                                                              const float* __restrict__ w,
-                                                              float* __restrict__ y, int D, float eps,
-                                                              int fast) {
+template <int NT>
+__global__ __launch_bounds__(NT) void rmsnorm_kernel(const float* __restrict__ x, const float* __restrict__ w,
+                                                     float* __restrict__ y, int D, float eps, int fast) {
   extern __shared__ float4 sq4[];
   __shared__ float inv_s;
   __shared__ SeqSumScratch seq;
   const int t = blockIdx.x, tid = threadIdx.x;
   const float* xt = x + (size_t)t * D;
   if (fast) {
-    // the row's first float4 a thread and its weights stay in registers
-    const bool in0 = tid < D / 4;
+    // 512 threads: the row's first float4 a thread and its weights stay in
+    // registers
+    constexpr int kept = NT == 512 ? NT : 0;
+    const bool in0 = tid < min(kept, D / 4);
     const float4 v0 = in0 ? reinterpret_cast<const float4*>(xt)[tid] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     f32x4_any w0 = {1.0f, 1.0f, 1.0f, 1.0f};
     if (in0 && w) w0 = reinterpret_cast<const f32x4_any*>(w)[tid];
     if (in0) sq4[tid] = make_float4(v0.x * v0.x, v0.y * v0.y, v0.z * v0.z, v0.w * v0.w);
-    for (int i = tid + kRmsThreads; i < D / 4; i += kRmsThreads) {
+    for (int i = tid + kept; i < D / 4; i += NT) {
       const float4 v = reinterpret_cast<const float4*>(xt)[i];
       sq4[i] = make_float4(v.x * v.x, v.y * v.y, v.z * v.z, v.w * v.w);
     }
     __syncthreads();
-    const float acc = block_seq_sum<kRmsThreads>(reinterpret_cast<const float*>(sq4), D, seq);
+    const float acc = block_seq_sum<NT>(reinterpret_cast<const float*>(sq4), D, seq);
     const float inv = 1.0f / sqrtf(acc / (float)D + eps);
     float* yt = y + (size_t)t * D;
     if (in0) {
@@ -579,7 +582,7 @@ __global__ __launch_bounds__(kRmsThreads) void rmsnorm_kernel(const float* __res
       const f32x4_any o = {n0 * w0[0], n1 * w0[1], n2 * w0[2], n3 * w0[3]};
       reinterpret_cast<f32x4_any*>(yt)[tid] = o;
     }
-    for (int i = 4 * kRmsThreads + tid; i < D; i += kRmsThreads) {
+    for (int i = 4 * kept + tid; i < D; i += NT) {
       const float v = xt[i] * inv;
       yt[i] = v * (w ? w[i] : 1.0f);
     }
@@ -587,7 +590,8 @@ __global__ __launch_bounds__(kRmsThreads) void rmsnorm_kernel(const float* __res
   }
   if (tid == 0) {
     float msq = 0.0f;
-    for (int i = 0; i < D; ++i) {
+#pragma unroll 16
+    for (int i = 0; i < D; ++i) {   // (16 loads in flight ahead of their adds)
       const float sq = xt[i] * xt[i];
       msq = msq + sq;
     }
@@ -596,7 +600,7 @@ __global__ __launch_bounds__(kRmsThreads) void rmsnorm_kernel(const float* __res
   }
   __syncthreads();
   const float inv = inv_s;
-  for (int i = tid; i < D; i += kRmsThreads) {
+  for (int i = tid; i < D; i += NT) {
     const float v = xt[i] * inv;
     y[(size_t)t * D + i] = v * (w ? w[i] : 1.0f);
   }
@@ -1092,18 +1096,24 @@ moe_status noalloc_scratch(uint8_t** out) {
 
 }  // namespace
 
-moe_status rmsnorm_dev(const float* x, const float* w, float* y, int T, int D, float eps) {
-  if (T <= 0) return MOE_OK;
-  const int fast = (D % 4 == 0) && aligned16(x) && (size_t)D * 4 <= kMaxLds;
+template <int NT>
+static moe_status launch_rmsnorm(const float* x, const float* w, float* y, int T, int D, float eps, int fast) {
   const size_t lds = fast ? (size_t)D * 4 : 0;
   if (lds > 65536) {
-    moe_status st = check_hip(hipFuncSetAttribute((const void*)rmsnorm_kernel,
+    moe_status st = check_hip(hipFuncSetAttribute((const void*)rmsnorm_kernel<NT>,
                                                   hipFuncAttributeMaxDynamicSharedMemorySize,
                                                   (int)lds), "rmsnorm LDS attribute");
     if (st) return st;
   }
-  hipLaunchKernelGGL(rmsnorm_kernel, dim3(T), dim3(kRmsThreads), lds, stream(), x, w, y, D, eps, fast);
+  hipLaunchKernelGGL(rmsnorm_kernel<NT>, dim3(T), dim3(NT), lds, stream(), x, w, y, D, eps, fast);
   return check_hip(hipGetLastError(), "rmsnorm launch");
+}
+
+moe_status rmsnorm_dev(const float* x, const float* w, float* y, int T, int D, float eps) {
+  if (T <= 0) return MOE_OK;
+  const int fast = (D % 4 == 0) && aligned16(x) && (size_t)D * 4 <= kMaxLds;
+  if (T <= 512 && (D >= 512 || T < 256)) return launch_rmsnorm<512>(x, w, y, T, D, eps, fast);
+  return launch_rmsnorm<256>(x, w, y, T, D, eps, fast);
 }
 
 void release_layer_scratch() { release_scratch_all(); }

@@ -302,6 +302,25 @@ def test_rmsnorm_dev(moehip):
         np.testing.assert_array_equal(bits(dy.download((T, D), np.float32)), bits(O.rmsnorm(x, w)))
 
 
+@pytest.mark.parametrize("T,D", [(255, 256), (256, 508), (256, 512), (512, 2052), (513, 4), (513, 2048), (600, 1001),
+                                 (520, 4100)])
+def test_rmsnorm_many_rows(moehip, T, D):
+    """512 threads a row up to 512 rows, 256 past them and for many short
+    rows; odd lengths; the special rows of the sums among the others."""
+    x = O.normal(T * D, 7 + D, 0.0, 2.0).reshape(T, D)
+    n = min(D, 2048)
+    x[T - 6:, :n] = _seq_sum_rows()[:, :n]
+    w = O.normal(D, 8 + D, 1.0, 0.1)
+    dx, dw, dy = (moehip.DeviceBuffer.from_array(x), moehip.DeviceBuffer.from_array(w),
+                  moehip.DeviceBuffer(x.nbytes))
+    moehip.check(moehip.lib().moe_rmsnorm_dev(dx.ptr, dw.ptr, dy.ptr, T, D, 1e-6))
+    with np.errstate(all="ignore"):
+        want = O.rmsnorm(x, w)
+    got, nan = dy.download((T, D), np.float32), np.isnan(want)
+    np.testing.assert_array_equal(np.isnan(got), nan)
+    np.testing.assert_array_equal(bits(got)[~nan], bits(want)[~nan])
+
+
 def _seq_sum_rows():
     """Rows whose sequential sum of squares defeats the segment estimates of
     block_seq_sum in different ways (every path of its stitching runs)."""
