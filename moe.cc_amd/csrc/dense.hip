@@ -865,23 +865,24 @@ __device__ void heads_prep(float* v0, float* v1, const float* w0, const float* w
   }
 }
 
-// kHeadRows consecutive (token, head) rows of [Q | K | V] a block (row q is
-// head q % (nq + 2 nkv) of token q / (nq + 2 nkv), hd wide): q/k rows through
-// the per-head RMSNorm and RoPE of heads_prep at position pos0 + t (Q in
-// place, K to the cache), V rows to the cache unchanged.  One lane a row runs
-// its sequential sum of squares, 16 rows side by side (one row a block left
-// the chip waiting on 20,480 such chains: 512 tokens, 40 heads of 128, 18.6 ->
-// 8.9 us).
-constexpr int kHeadRows = 16;
-
-__global__ __launch_bounds__(256) void heads_kernel(HeadArgs a) {
-  extern __shared__ float hrow[];   // [kHeadRows][hd + 4] rows, then the same of squares
-  __shared__ float inv_s[kHeadRows];
-  constexpr int RW = kHeadRows / 4;   // rows a wave
+// 4 RW consecutive (token, head) rows of [Q | K | V] a block (row q is head q %
+// (nq + 2 nkv) of token q / (nq + 2 nkv), hd wide): q/k rows through the
+// per-head RMSNorm and RoPE of heads_prep at position pos0 + t (Q in place, K
+// to the cache), V rows to the cache unchanged.  Latency: one lane a row runs
+// its sequential sum of squares, the rows of a block side by side.  RW = 4 once
+// its blocks fill the chip: one row a block left it waiting on 20,480 such
+// chains (512 tokens, 40 heads of 128, 18.1 -> 8.4 us); RW = 1 below, where
+// more rows a block only add to the wait (3 tokens 6.1 -> 4.7 us, 40 tokens
+// 5.5 -> 4.8).
+template <int RW>
+__global__ __launch_bounds__(256, RW == 4 ? 5 : 1) void heads_kernel(HeadArgs a) {
+  constexpr int NR = 4 * RW;
+  extern __shared__ float hrow[];   // [NR][hd + 4] rows, then the same of squares
+  __shared__ float inv_s[NR];
   const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
   const int hd = a.hd, d2 = hd / 2, LD = hd + 4, H = a.nq + 2 * a.nkv;
-  const long long q0 = (long long)blockIdx.x * kHeadRows, nrow = (long long)a.T * H;
-  float* sq = hrow + kHeadRows * LD;
+  const long long q0 = (long long)blockIdx.x * NR, nrow = (long long)a.T * H;
+  float* sq = hrow + NR * LD;
   float* row[RW];
   int t[RW], h[RW];
 #pragma unroll
@@ -901,8 +902,19 @@ __global__ __launch_bounds__(256) void heads_kernel(HeadArgs a) {
       sq[(wave * RW + i) * LD + d] = v[i] * v[i];
     }
   }
+  // weights, cosine and sine of a lane's pair of columns; the first pair's
+  // are requested here (RW = 1: four rows' would cost a block its neighbour,
+  // 512 tokens 8.4 -> 10.1 us)
+  struct Pair { float w0, w1, c, s; };
+  auto fetch = [&](int i, int d) {
+    const float* w = h[i] < a.nq ? a.q_norm : a.k_norm;
+    const size_t at = (size_t)(a.pos0 + t[i]) * d2 + d;
+    return Pair{w ? w[d] : 1.0f, w ? w[d + d2] : 1.0f, a.rope_cos[at], a.rope_sin[at]};
+  };
+  Pair first{};
+  if (RW == 1 && lane < d2) first = fetch(0, lane);
   __syncthreads();
-  if ((int)threadIdx.x < kHeadRows) {
+  if ((int)threadIdx.x < NR) {
     const float msq = chain_sum(0.0f, sq + threadIdx.x * LD, hd / 4);
     inv_s[threadIdx.x] = 1.0f / sqrtf(msq / (float)hd + a.eps);
   }
@@ -917,19 +929,19 @@ __global__ __launch_bounds__(256) void heads_kernel(HeadArgs a) {
       for (int d = lane; d < hd; d += kWave) dst[d] = v[d];
       continue;
     }
-    const float* w = h[i] < a.nq ? a.q_norm : a.k_norm;
+    const bool normed = (h[i] < a.nq ? a.q_norm : a.k_norm) != nullptr;
     float* out = h[i] < a.nq ? row[i] : a.kc + ((size_t)(h[i] - a.nq) * a.max_seq + pos) * hd;
     const float inv = inv_s[wave * RW + i];
     for (int d = lane; d < d2; d += kWave) {
+      const Pair p = RW == 1 && d == lane ? first : fetch(i, d);
       float e = v[d], o = v[d + d2];
-      if (w) {
+      if (normed) {
         e = e * inv;
         o = o * inv;
-        e = e * w[d];
-        o = o * w[d + d2];
+        e = e * p.w0;
+        o = o * p.w1;
       }
-      const float c = a.rope_cos[(size_t)pos * d2 + d], s = a.rope_sin[(size_t)pos * d2 + d];
-      const float ec = e * c, os = o * s, oc = o * c, es = e * s;
+      const float ec = e * p.c, os = o * p.s, oc = o * p.c, es = e * p.s;
       out[d] = ec - os;
       out[d + d2] = oc + es;
     }
@@ -2000,15 +2012,20 @@ moe_status embed_rows(const int32_t* ids, int T, const float* emb, int V, int D,
   return check_hip(hipGetLastError(), "embed launch");
 }
 
+template <int RW>
+static moe_status launch_heads(const HeadArgs& a, long long rows, hipStream_t s) {
+  const size_t lds = (size_t)2 * 4 * RW * (a.hd + 4) * 4;
+  moe_status st = set_lds(heads_kernel<RW>, lds, "heads LDS attribute");
+  if (st) return st;
+  hipLaunchKernelGGL(heads_kernel<RW>, dim3((unsigned)((rows + 4 * RW - 1) / (4 * RW))), dim3(256), lds, s, a);
+  return check_hip(hipGetLastError(), "heads launch");
+}
+
 moe_status heads_norm_rope(const HeadArgs& a, hipStream_t s) {
   if (a.T <= 0) return MOE_OK;
   if (a.hd > kMaxHd || (a.hd & 1)) return set_error(MOE_ERR_ARG, "head_dim %d unsupported", a.hd);
-  const size_t lds = (size_t)2 * kHeadRows * (a.hd + 4) * 4;
-  moe_status st = set_lds(heads_kernel, lds, "heads LDS attribute");
-  if (st) return st;
   const long long rows = (long long)a.T * (a.nq + 2 * a.nkv);
-  hipLaunchKernelGGL(heads_kernel, dim3((unsigned)((rows + kHeadRows - 1) / kHeadRows)), dim3(256), lds, s, a);
-  return check_hip(hipGetLastError(), "heads launch");
+  return rows < 4096 ? launch_heads<1>(a, rows, s) : launch_heads<4>(a, rows, s);
 }
 
 moe_status attention_rows(const AttnArgs& a, hipStream_t s) {

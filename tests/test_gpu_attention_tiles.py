@@ -19,7 +19,9 @@ def bits(a):
 # (head_dim, query heads, KV heads, cache length, prompt chunks)
 CASES = [(128, 8, 2, 131, (5, 16, 32, 17, 33, 28)), (64, 6, 2, 70, (31, 33, 6)), (32, 5, 1, 67, (32, 35)),
          (96, 16, 16, 200, (129, 65, 5)), (68, 3, 3, 65, (64,)), (256, 8, 1, 150, (15, 128)),
-         (512, 2, 1, 49, (33, 16)), (4, 8, 8, 300, (257, 6, 37))]
+         (512, 2, 1, 49, (33, 16)), (4, 8, 8, 300, (257, 6, 37)),
+         # 4095 and 4224 head rows, on both sides of the head kernel's rule
+         (64, 15, 15, 92, (91,)), (512, 16, 16, 90, (88,))]
 
 
 @pytest.mark.parametrize("hd,nq,nkv,max_seq,chunks", CASES)
