@@ -1478,28 +1478,32 @@ __global__ __launch_bounds__(256) void attn_softmax_rows_kernel(AttnArgs a, int 
   }
 }
 
-// Weighted V sums of query rows t0 .. t0 + 31 of one head for dimensions 64
-// blockIdx.y ..; wave w: rows 16 (w % 2) .., dimensions 32 (w /
-// 2) ...  out = (((0 + p_0 v_0) + p_1 v_1) + ...) over a row's n = pos0 + t + 1
+// Weighted V sums of query rows t0 .. t0 + 15 of one head for dimensions 64
+// blockIdx.y ..; wave w: dimensions 16 w .. of those.  out = (((0 + p_0 v_0) + p_1 v_1) + ...) over a row's n = pos0 + t + 1
 // positions: chunks of kPvCh positions of p (rows a.ss apart) and V stream
 // through two LDS buffers; a product past the row's n counts as +0, which
 // leaves its chain unchanged (a chain from +0 is never -0).  The longest
-// rows' blocks come first in the grid.
-constexpr int kPvCh = 32;
+// rows' blocks come first in the grid.  One 16 x 16 tile of products a step and
+// wave: two (32 rows a block) double the chain of a launch that a few rows
+// leave waiting, and cost the full chip a block a CU in registers (32 / 4 heads
+// of 128, 8 rows at position 1000: 32.2 -> 20.9 us, 64 rows 36.7 -> 24.4, 512
+// rows at 1000 .. 72.6 -> 68.7).
+constexpr int kPvCh = 32, kPvR = 16;
 
-__global__ __launch_bounds__(256, 3) void attn_pv_qt_kernel(AttnArgs a) {
+__global__ __launch_bounds__(256, 4) void attn_pv_qt_kernel(AttnArgs a) {
   constexpr int PS = kPvCh / 4, VS = 16;                  // 16-byte slots of a p row, a V row (64 dimensions)
-  constexpr int NP = kSq * PS / 64, NV = kPvCh * VS / 64; // load instructions
-  static_assert(NP == 4 && NV == 8, "whole instructions per wave");
-  __shared__ float4 lds4[2][kSq * PS + kPvCh * VS];
+  constexpr int NP = kPvR * PS / 64, NV = kPvCh * VS / 64; // load instructions
+  static_assert(NP == 2 && NV == 8, "one of the first two waves, two of every wave");
+  __shared__ float4 lds4[2][kPvR * PS + kPvCh * VS];
   const int hd = a.hd, h = attn_head(blockIdx.x, a.nq), d0 = blockIdx.y * 64;
-  const int t0 = ((int)gridDim.z - 1 - (int)blockIdx.z) * kSq;
+  const int t0 = ((int)gridDim.z - 1 - (int)blockIdx.z) * kPvR;
   const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  const int b = lane / 16, j = lane % 16, wx = wave % 2, wn = wave / 2;
-  const int nmax = min(a.pos0 + t0 + kSq, a.pos0 + a.T);  // positions of the last row
+  const int b = lane / 16, j = lane % 16;
+  const int nmax = min(a.pos0 + t0 + kPvR, a.pos0 + a.T);  // positions of the last row
   const int nc = (nmax + kPvCh - 1) / kPvCh;
   const int kvh = h / (a.nq / a.nkv);
-  // instruction `wave` loads p rows (8 each), 4 + wave and 8 + wave V rows (4 each)
+  // instruction `wave` < NP loads p rows (8 each), NP + wave and NP + 4 + wave V
+  // rows (4 each)
   const int prow = 8 * wave + lane / PS, pcol = 4 * ((lane % PS) ^ ((prow >> 1) & 7));
   const float* psrc = a.S + ((size_t)h * a.T + min(t0 + prow, a.T - 1)) * a.ss + pcol;
   const float* vbase = a.vc + (size_t)kvh * a.max_seq * hd;
@@ -1514,63 +1518,52 @@ __global__ __launch_bounds__(256, 3) void attn_pv_qt_kernel(AttnArgs a) {
   auto load = [&](int c, int half) {
     uint8_t* l = reinterpret_cast<uint8_t*>(lds4[half]);
     const int c0 = c * kPvCh;
-    lds_load16(c0 + pcol < a.ss ? psrc + c0 : kDenseZero, l + wave * 1024);
+    if (wave < NP) lds_load16(c0 + pcol < a.ss ? psrc + c0 : kDenseZero, l + wave * 1024);
 #pragma unroll
     for (int v = 0; v < 2; ++v)
       lds_load16(vcol[v] < hd ? vbase + (size_t)min(c0 + vrow[v], nmax - 1) * hd + vcol[v] : kDenseZero,
-                 l + (4 + wave + 4 * v) * 1024);
+                 l + (NP + wave + 4 * v) * 1024);
   };
-  const int nlo = a.pos0 + t0 + 16 * wx + 1, nhi = nlo + 15;   // positions of the wave's rows
-  float acc[2][4] = {};
+  const int nlo = a.pos0 + t0 + 1, nhi = nlo + 15;   // positions of the first and the last row
+  float acc[4] = {};
   load(0, 0);
   for (int c = 0; c < nc; ++c) {
     stage_sync<0>();
     if (c + 1 < nc) load(c + 1, (c + 1) & 1);
-    const float4* P = lds4[c & 1] + (16 * wx + j) * PS;
-    const float* V = reinterpret_cast<const float*>(lds4[c & 1] + kSq * PS);
+    const float4* P = lds4[c & 1] + j * PS;
+    const float* V = reinterpret_cast<const float*>(lds4[c & 1] + kPvR * PS);
 #pragma unroll
     for (int g = 0; g < kPvCh / 16; ++g) {
       const int pos = c * kPvCh + 16 * g;
       if (pos >= nhi) break;
       const float4 x = P[(4 * g + b) ^ ((j >> 1) & 7)];
-      float4 w[2];
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        const float* v = V + (16 * g + 4 * b) * 64 + 4 * ((4 * (2 * wn + t) + j / 4) ^ (4 * b)) + j % 4;
-        w[t] = make_float4(v[0], v[64], v[128], v[192]);
-      }
-      const bool masked = pos + 16 > nlo;
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        v16f p[4];
-        mfma_products(x, w[t], p);
-        if (masked) {
-          int left = a.pos0 + t0 + 16 * wx + 4 * b + 1 - pos;   // row r: left + r positions from pos on
-          asm volatile("" : "+v"(left));   // (64 comparison masks kept for both tiles would spill)
-#pragma unroll
-          for (int k = 0; k < 16; ++k)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              const float q = p[k % 4][4 * (k / 4) + r];
-              p[k % 4][4 * (k / 4) + r] = k < left + r ? q : 0.0f;
-            }
-        }
-        __builtin_amdgcn_sched_barrier(0);
+      const float* v = V + (16 * g + 4 * b) * 64 + 4 * ((4 * wave + j / 4) ^ (4 * b)) + j % 4;
+      const float4 w = make_float4(v[0], v[64], v[128], v[192]);
+      v16f p[4];
+      mfma_products(x, w, p);
+      if (pos + 16 > nlo) {
+        const int left = nlo + 4 * b - pos;   // row r: left + r positions from pos on
 #pragma unroll
         for (int k = 0; k < 16; ++k)
 #pragma unroll
-          for (int r = 0; r < 4; ++r) acc[t][r] = acc[t][r] + p[k % 4][4 * (k / 4) + r];
-        __builtin_amdgcn_sched_barrier(0);
+          for (int r = 0; r < 4; ++r) {
+            const float q = p[k % 4][4 * (k / 4) + r];
+            p[k % 4][4 * (k / 4) + r] = k < left + r ? q : 0.0f;
+          }
       }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int k = 0; k < 16; ++k)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[r] = acc[r] + p[k % 4][4 * (k / 4) + r];
+      __builtin_amdgcn_sched_barrier(0);
     }
   }
 #pragma unroll
-  for (int t = 0; t < 2; ++t)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int tok = t0 + 16 * wx + 4 * b + r, d = d0 + 16 * (2 * wn + t) + j;
-      if (tok < a.T && d < hd) a.H[(size_t)tok * a.nq * hd + (size_t)h * hd + d] = acc[t][r];
-    }
+  for (int r = 0; r < 4; ++r) {
+    const int tok = t0 + 4 * b + r, d = d0 + 16 * wave + j;
+    if (tok < a.T && d < hd) a.H[(size_t)tok * a.nq * hd + (size_t)h * hd + d] = acc[r];
+  }
 }
 
 // ---------------------------------------------------------------- misc
@@ -2050,7 +2043,8 @@ moe_status attention_rows(const AttnArgs& a, hipStream_t s) {
     hipLaunchKernelGGL(attn_softmax_rows_kernel, dim3((unsigned)a.nq, (unsigned)((a.T + R - 1) / R)), dim3(256), lds_m,
                        s, a, R);
     if ((st = check_hip(hipGetLastError(), "softmax rows launch"))) return st;
-    hipLaunchKernelGGL(attn_pv_qt_kernel, dim3((unsigned)a.nq, (unsigned)((a.hd + 63) / 64), qg), dim3(256), 0, s, a);
+    hipLaunchKernelGGL(attn_pv_qt_kernel, dim3((unsigned)a.nq, (unsigned)((a.hd + 63) / 64),
+                                               (unsigned)((a.T + kPvR - 1) / kPvR)), dim3(256), 0, s, a);
     return check_hip(hipGetLastError(), "softmax/pv launch");
   }
   const int nmax = a.pos0 + a.T;   // positions of the last row
