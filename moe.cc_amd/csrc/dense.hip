@@ -1306,23 +1306,25 @@ __device__ __forceinline__ int attn_head(int x, int nq) {
   return nq % 8 ? x : x % 8 * (nq / 8) + x / 8;
 }
 
-// Scores of query rows t0 .. t0 + 31 of one head against
-// kSkt tiles of 32 keys from 128 blockIdx.y on; wave w: rows 16 (w %
-// 2) .., keys 16 (w / 2) .. of each tile.  The queries stay in LDS, the key
+// Scores of query rows t0 .. t0 + 31 of one head against `tiles` tiles of 32
+// keys from 32 tiles blockIdx.y on; wave w: rows 16 (w % 2) .., keys 16 (w / 2)
+// .. of each tile.  The queries stay in LDS, the key
 // tiles stream through a ring of D buffers in stages of 64 columns (nh stages
 // a tile, columns past hd zero), so that only a block's first loads are waited
-// for (one tile a block: 45 us at 512 rows, most of it blocks waiting for
-// their own two loads).  q must already be normed and rotated (heads_kernel).
+// for (512 rows, one tile a block: 45 us, most of it blocks waiting for their
+// own two loads; with fewer blocks than the chip
+// holds the wait for more tiles is longer than that one: 8 rows at position 250
+// 11.3 -> 6.2 us, 512 rows of 4 heads 17.1 -> 16.0).  q must already be normed and rotated (heads_kernel).
 // S rows (head, token) are a.ss apart; key <= pos0 + t only is written.
-constexpr int kSq = 32, kSk = 32, kSkt = 4;
+constexpr int kSq = 32, kSk = 32, kSktMax = 4;
 constexpr int kSkD = 3;
 constexpr int kStageB = 32 * 64 * 4;   // bytes of 32 rows x 64 columns
 
-__global__ __launch_bounds__(256, 4) void attn_scores_qt_kernel(AttnArgs a) {
+__global__ __launch_bounds__(256, 4) void attn_scores_qt_kernel(AttnArgs a, int tiles) {
   constexpr int SL = 16, NL = 2;   // 16-byte slots of a row; load instructions of a stage per wave
   extern __shared__ float4 sq4[];  // [nh] query stages, [kSkD] key stages
   const int hd = a.hd, nh = (hd + 63) / 64;
-  const int h = attn_head(blockIdx.x, a.nq), tk0 = blockIdx.y * (kSk * kSkt);
+  const int h = attn_head(blockIdx.x, a.nq), tk0 = blockIdx.y * (kSk * tiles);
   const int t0 = ((int)gridDim.z - 1 - (int)blockIdx.z) * kSq;
   const int Pmax = min(a.pos0 + t0 + kSq, a.pos0 + a.T) - 1;
   if (tk0 > Pmax) return;   // every key of the block is masked (uniform)
@@ -1330,7 +1332,7 @@ __global__ __launch_bounds__(256, 4) void attn_scores_qt_kernel(AttnArgs a) {
   const int b = lane / 16, j = lane % 16, wx = wave % 2, wn = wave / 2;
   const int kvh = h / (a.nq / a.nkv);
   const float* kbase = a.kc + (size_t)kvh * a.max_seq * hd;
-  const int steps = min(kSkt, (Pmax - tk0) / kSk + 1) * nh;
+  const int steps = min(tiles, (Pmax - tk0) / kSk + 1) * nh;
   uint8_t* qlds = reinterpret_cast<uint8_t*>(sq4);
   uint8_t* klds = qlds + nh * kStageB;
   // instruction v of a stage: rows 4 (wave + 4v) + lane / 16
@@ -2028,11 +2030,15 @@ moe_status attention_rows(const AttnArgs& a, hipStream_t s) {
   if (a.T > 4 && !a.fuse_heads && a.nkv > 0 && a.nq % a.nkv == 0 && a.ss % 4 == 0 && al16(a.qkv) &&
       a.ld % 4 == 0 && !getenv("MOEHIP_ATTN_ROWWISE")) {
     const unsigned qg = (unsigned)((a.T + kSq - 1) / kSq);
-    const dim3 sg((unsigned)a.nq, (unsigned)((a.pos0 + a.T + kSk * kSkt - 1) / (kSk * kSkt)), qg);
+    const int keys = a.pos0 + a.T;
+    // fewer key tiles a block where four would leave under 1024 blocks
+    int tiles = kSktMax;
+    while (tiles > 1 && (long long)a.nq * qg * ((keys + kSk * tiles - 1) / (kSk * tiles)) < 1024) tiles /= 2;
+    const dim3 sg((unsigned)a.nq, (unsigned)((keys + kSk * tiles - 1) / (kSk * tiles)), qg);
     const size_t lds_s = (size_t)((a.hd + 63) / 64 + kSkD) * kStageB;
     moe_status st;
     if ((st = set_lds(attn_scores_qt_kernel, lds_s, "scores LDS attribute"))) return st;
-    hipLaunchKernelGGL(attn_scores_qt_kernel, sg, dim3(256), lds_s, s, a);
+    hipLaunchKernelGGL(attn_scores_qt_kernel, sg, dim3(256), lds_s, s, a, tiles);
     if ((st = check_hip(hipGetLastError(), "scores launch"))) return st;
     // rows a block: 16, fewer where they would not fit two blocks a CU
     int R = kSmRowsMax;
