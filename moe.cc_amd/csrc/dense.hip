@@ -1289,13 +1289,14 @@ __global__ __launch_bounds__(kPvThreads) void attn_softmax_pv_kernel(AttnArgs a)
 // ---- many query rows (prefill) ----
 //
 // The one-row kernels above read the whole key / value prefix once per query
-// row; these read it once per 32 rows, with the products on the matrix cores
-// and the chains' adds on the VALU as in dense_mfma_kernel (its operand
-// layout: lane (b, j) = (lane / 16, lane % 16), MFMA c of 16 columns has
+// row; these read it once per 32 (scores) or 16 rows (V sums), with the
+// products on the matrix cores and the chains' adds on the VALU as in
+// dense_mfma_kernel (its operand layout: lane (b, j) = (lane / 16, lane % 16), MFMA c of 16 columns has
 // column 4b + c in block b, result register 4b' + r of MFMA c the product of
 // chain r and column 4b' + c).  Same chains, same order: bit-identical
-// results.  512 rows, 32 / 4 heads of 128: scores 71 -> 32 us, V sums 74 -> 26
-// (15 of each are the products and adds at 4.3 clocks per 64), softmax 18.
+// results.  512 rows from position 0, 32 / 4 heads of 128: scores 71 -> 32 us, V
+// sums 74 -> 25 (15 of each are the products and adds at 4.3 clocks per 64),
+// softmax 16.
 
 // The head of block x of a grid whose x runs over the nq heads: blocks are
 // dealt to the 8 XCDs in turn, so XCD k takes heads k nq/8 .. and a KV head's
@@ -1408,11 +1409,14 @@ __global__ __launch_bounds__(256, 4) void attn_scores_qt_kernel(AttnArgs a, int 
 
 // Softmax of the score rows, in place (test_model_trace.c:411-420): a block
 // takes R query rows of a head, n = pos0 + t + 1 scores each, staged in LDS
-// (the longest rows' blocks first, those of one length spread over the CUs); max per row by one wave (order-free; a NaN first score wins, as in
+// (the longest rows' blocks first, those of one length spread over the CUs);
+// max per row by one wave (order-free; a NaN first score wins, as in
 // attn_softmax_pv_kernel), e = expf(s - m), then lane i of wave 0 runs row
-// i's sum chain -- R chains a wave instead of one -- and p = e * (1 / (sum +
-// 1e-9)) goes back over the scores.
-constexpr int kSmRowsMax = 16;
+// i's sum chain, and p = e * (1 / (sum + 1e-9)) goes back over the scores.  A
+// row a wave: 16 rows a block left each wave four rows to exponentiate one
+// after another (32 heads: 16 rows at position 250 9.6 -> 5.2 us, 8 at 1000 14.5
+// -> 10.2, 512 at 0 .. 1500 49 -> 36; two rows 51, one row 80).
+constexpr int kSmRowsMax = 4;
 
 // Floats of a staged row: whole 256-float load instructions, and four so that
 // the 16 lanes of a chain read meet different banks.
@@ -2040,9 +2044,9 @@ moe_status attention_rows(const AttnArgs& a, hipStream_t s) {
     if ((st = set_lds(attn_scores_qt_kernel, lds_s, "scores LDS attribute"))) return st;
     hipLaunchKernelGGL(attn_scores_qt_kernel, sg, dim3(256), lds_s, s, a, tiles);
     if ((st = check_hip(hipGetLastError(), "scores launch"))) return st;
-    // rows a block: 16, fewer where they would not fit two blocks a CU
+    // rows a block: 4, fewer where they would not fit two blocks a CU
     int R = kSmRowsMax;
-    const size_t row_b = (size_t)sm_row_floats(a.pos0 + a.T) * 4;
+    const size_t row_b = (size_t)sm_row_floats(keys) * 4;
     while (R > 1 && R * row_b > 72 * 1024) R /= 2;
     const size_t lds_m = R * row_b;
     if ((st = set_lds(attn_softmax_rows_kernel, lds_m, "softmax rows LDS attribute"))) return st;
