@@ -1134,21 +1134,21 @@ __global__ __launch_bounds__(64) void attn_scores_kernel(AttnArgs a) {
   }
 }
 
-constexpr int kPvThreads = 256;
+constexpr int kPvThreads = 256, kPvDpb = 16;
 
 // Softmax of the n = pos0 + t + 1 scores of (t, h) and the weighted V sum
-// for head dimensions DPB*g .. DPB*g + DPB - 1 (test_model_trace.c:408-426):
+// for head dimensions DPB*g .. DPB*g + DPB - 1 (test_model_trace.c:408-426), up
+// to four query rows:
 //   m = S[0], then every larger score (a NaN S[0] stays; later NaNs never
 //   win); e_i = expf(S_i - m); sum = (((0 + e_0) + e_1) + ...) (the
-//   sequential sum: one chain, or block_seq_sum for the long rows of
-//   prefill);
+//   sequential sum: one chain, or block_seq_sum for long rows);
 //   p_i = e_i * (1 / (sum + 1e-9)); out_d = (((0 + p_0 v_0d) + p_1 v_1d) + ...).
 // The weighted sum runs over chunks of CH positions: every thread forms
 // products p_i * v_id of the chunk into a transposed LDS tile [d][i] (the
 // next chunk's V loads already in flight), then lanes d < DPB sum their row
 // with pure dependent adds.  Products past n are 0 * 0 = +0 (no-ops).
-template <int DPB>
 __global__ __launch_bounds__(kPvThreads) void attn_softmax_pv_kernel(AttnArgs a) {
+  constexpr int DPB = kPvDpb;
   constexpr int CH = 16384 / DPB;                  // positions per chunk
   constexpr int Q4 = DPB / 4;                      // float4 per position
   constexpr int NL = CH * Q4 / kPvThreads;         // float4 per thread per chunk
@@ -2031,8 +2031,9 @@ moe_status attention_rows(const AttnArgs& a, hipStream_t s) {
   if (a.T <= 0) return MOE_OK;
   if (a.hd % 4 || a.hd > kMaxHd) return set_error(MOE_ERR_ARG, "attention: head_dim %d", a.hd);
   if (a.fuse_heads && a.T != 1) return set_error(MOE_ERR_ARG, "attention: fused heads need T == 1");
-  if (a.T > 4 && !a.fuse_heads && a.nkv > 0 && a.nq % a.nkv == 0 && a.ss % 4 == 0 && al16(a.qkv) &&
-      a.ld % 4 == 0 && !getenv("MOEHIP_ATTN_ROWWISE")) {
+  if (a.T > 4) {
+    if (a.nkv <= 0 || a.nq % a.nkv || a.ss % 4 || a.ld % 4 || !al16(a.qkv))
+      return set_error(MOE_ERR_ARG, "attention: many rows need whole head groups and 16-byte aligned rows");
     const unsigned qg = (unsigned)((a.T + kSq - 1) / kSq);
     const int keys = a.pos0 + a.T;
     // fewer key tiles a block where four would leave under 1024 blocks
@@ -2074,17 +2075,10 @@ moe_status attention_rows(const AttnArgs& a, hipStream_t s) {
   }
   if ((st = check_hip(hipGetLastError(), "scores launch"))) return st;
   const size_t es_f = (size_t)((a.max_seq + 3) & ~3);
-  if (a.T <= 4) {
-    const size_t lds_p = (es_f + 16 * (16384 / 16 + 4)) * 4;
-    if ((st = set_lds(attn_softmax_pv_kernel<16>, lds_p, "softmax/pv LDS attribute"))) return st;
-    hipLaunchKernelGGL(attn_softmax_pv_kernel<16>, dim3((unsigned)((a.hd + 15) / 16), (unsigned)a.nq, (unsigned)a.T),
-                       dim3(kPvThreads), lds_p, s, ax);
-  } else {
-    const size_t lds_p = (es_f + 128 * (16384 / 128 + 4)) * 4;
-    if ((st = set_lds(attn_softmax_pv_kernel<128>, lds_p, "softmax/pv LDS attribute"))) return st;
-    hipLaunchKernelGGL(attn_softmax_pv_kernel<128>, dim3((unsigned)((a.hd + 127) / 128), (unsigned)a.nq, (unsigned)a.T),
-                       dim3(kPvThreads), lds_p, s, ax);
-  }
+  const size_t lds_p = (es_f + kPvDpb * (16384 / kPvDpb + 4)) * 4;
+  if ((st = set_lds(attn_softmax_pv_kernel, lds_p, "softmax/pv LDS attribute"))) return st;
+  hipLaunchKernelGGL(attn_softmax_pv_kernel, dim3((unsigned)((a.hd + kPvDpb - 1) / kPvDpb), (unsigned)a.nq, (unsigned)a.T),
+                     dim3(kPvThreads), lds_p, s, ax);
   return check_hip(hipGetLastError(), "softmax/pv launch");
 }
 

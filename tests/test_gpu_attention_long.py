@@ -12,12 +12,12 @@ run the kernels' multi-block paths at configs[4]'s head geometry
 * 70 single-token decode steps across two more key-block boundaries (320,
   384), each step's logits checked;
 * a second prompt chunk at position 390 (query tiles at pos0 > 0);
-* the per-row kernels for many rows (MOEHIP_ATTN_ROWWISE), which the
-  library takes when the query-tiled kernel's LDS rows do not fit;
+* the one-row kernels with two to four rows, past several chunks of V;
 * 2060 cached positions (decode's scores no longer fit in registers,
-  several 1024-position V chunks) and 4650 (the query-tiled kernel's LDS
-  limit: the rowwise kernels take over by themselves), with 4 / 1 query
-  heads so that the CPU oracle stays fast.
+  several 1024-position V chunks) and 4650, where four score rows no longer fit
+  a softmax block's LDS share (two a block), with 4 / 1 query heads so that the
+  CPU oracle stays fast; narrow heads to the longest cache, 16384 positions
+  (one row a block from 8961 on).
 
 Bar: bit-exact against oracle/model_oracle.c's KV-cached forward, itself
 pinned to the compiled reference's model_forward_f32 (tests/golden/
@@ -72,25 +72,25 @@ def test_long_prompt_decode_and_second_chunk(moehip):
     m.close()
 
 
-def test_long_rowwise_kernels(moehip, monkeypatch):
-    """The per-row score and softmax / V kernels for many rows (the path
-    taken when the query-tiled kernel's LDS rows do not fit): a 300-token
-    prompt (three 128-position V chunks, the block-parallel exact sum of
-    each row's exponentials), then a 9-token chunk and decode steps."""
-    print("attention long: rowwise kernels, prompt 300", flush=True)
-    monkeypatch.setenv("MOEHIP_ATTN_ROWWISE", "1")
+def test_long_rowwise_kernels(moehip):
+    """The one-row score and softmax / V kernels with two to four rows at
+    positions 296-318 (the block-parallel exact sum of each row's exponentials,
+    three 128-position pieces of V), then decode steps."""
+    print("attention long: two to four rows at 296", flush=True)
     tm = O.TinyModel(seed=43, **GEOM)
     m = moehip.model_from_tiny(tm, max_seq=400)
     cache = tm.new_cache(400)
-    ids = (O.uniform_u32(300, 143) % tm.V).astype(np.int32)
+    ids = (O.uniform_u32(296, 143) % tm.V).astype(np.int32)
     want = tm.forward_kv(ids, 0, cache)
     got, nxt = m.forward(ids)
-    _check(got, want, "rowwise prompt 300")
-    chunk = (O.uniform_u32(9, 144) % tm.V).astype(np.int32)
-    want = tm.forward_kv(chunk, 300, cache)
-    got, nxt = m.forward(chunk)
-    _check(got, want, "rowwise chunk at 300")
-    pos = 309
+    _check(got, want, "prompt 296")
+    pos = 296
+    for T in (4, 3, 2, 4, 4, 3, 2):
+        chunk = (O.uniform_u32(T, 144 + pos) % tm.V).astype(np.int32)
+        want = tm.forward_kv(chunk, pos, cache)
+        got, nxt = m.forward(chunk)
+        _check(got, want, f"{T} rows at {pos}")
+        pos += T
     for step in range(12):
         want = tm.forward_kv([nxt], pos, cache)
         got, nxt = m.forward([nxt])
@@ -122,10 +122,8 @@ def test_context_2060(moehip):
 
 
 def test_context_past_tile_lds(moehip):
-    """A 4600-token prompt (query-tiled kernels at their largest), then a
-    50-token chunk at position 4600: 8 rows of 4652 scores no longer fit the
-    query-tiled kernel's LDS, so the library runs the per-row kernels on
-    its own; then decode steps."""
+    """A 4600-token prompt and a 50-token chunk behind it: past 4352 scores a
+    softmax block holds two rows instead of four; then decode steps."""
     print("attention long: prompt 4600 / chunk 50 / decode", flush=True)
     tm = O.TinyModel(D=128, L=1, hd=128, nq=1, nkv=1, dff=128, E=16, V=300, dtype=3, seed=45)
     max_seq = 4700
@@ -145,4 +143,23 @@ def test_context_past_tile_lds(moehip):
         got, nxt = m.forward([nxt])
         _check(got, want, f"decode at position {pos}")
         pos += 1
+    m.close()
+
+
+def test_context_to_the_longest_cache(moehip):
+    """A 9200-token prompt, chunks of 7 and 40 rows behind it (a softmax row of
+    more than 8960 scores: one row a block), a prompt to 16340 and chunks that
+    end at the longest cache, 16384 positions."""
+    print("attention long: 16384 positions", flush=True)
+    tm = O.TinyModel(D=64, L=1, hd=8, nq=1, nkv=1, dff=32, E=8, top_k=2, V=60, dtype=3, seed=46)
+    m = moehip.model_from_tiny(tm, max_seq=16384)
+    cache = tm.new_cache(16384)
+    pos = 0
+    for T in (9200, 7, 40, 7093, 39, 5):
+        ids = (O.uniform_u32(T, 150 + T) % tm.V).astype(np.int32)
+        want = tm.forward_kv(ids, pos, cache)
+        got, _ = m.forward(ids)
+        _check(got, want, f"{T} rows at {pos}")
+        pos += T
+    assert pos == 16384 == m.position
     m.close()
