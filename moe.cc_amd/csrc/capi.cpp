@@ -105,6 +105,19 @@ moe_status grow(void** buf, size_t* cap, size_t need) {
   return st;
 }
 
+// The pinned staging, allocated once; false where the host has none to give.
+bool pin_staging() {
+  for (void** b : {&g_pin_a, &g_pin_c}) {
+    if (*b) continue;
+    if (hipHostMalloc(b, kPinBytes, hipHostMallocDefault) != hipSuccess) {
+      *b = nullptr;
+      (void)hipGetLastError();   // the next launch check must not see it
+      return false;
+    }
+  }
+  return true;
+}
+
 // 64-bit digest of a host buffer: eight lanes, each folding two 8-byte words
 // and its state through one 64 x 64 -> 128 bit product (16 bytes a multiply),
 // the lanes' old states kept beside the product so that a zero factor loses no
@@ -556,10 +569,8 @@ void matmul_adaptive(const float* A, const float* W_fp32, const void* W_q_ptr, f
                          : dtype == 2 ? (size_t)N * (size_t)K
                                       : (size_t)N * (size_t)(K / 2) + (size_t)(K & 1);
   const size_t s_bytes = wq ? (size_t)N * sizeof(float) : 0;
-  const bool pin = a_bytes <= kPinBytes && c_bytes <= kPinBytes;
-  for (void** b : {&g_pin_a, &g_pin_c})
-    if (pin && !*b && check_hip(hipHostMalloc(b, kPinBytes, hipHostMallocDefault), "hipHostMalloc(staging)"))
-      die("matmul_adaptive staging");
+  // without pinned memory the copies wait, as they do past kPinBytes
+  const bool pin = a_bytes <= kPinBytes && c_bytes <= kPinBytes && pin_staging();
   void* dst = pin ? g_pin_c : (void*)C;
   // Weights seen before: the product starts on their cached copies, and the
   // host bytes are checked while it runs; the result only reaches C if they

@@ -1,6 +1,10 @@
 """The drop-in matmul_adaptive on weights it has seen before: the product
 starts on the cached device copy while the host bytes are checked, so a weight
 changed in place must still give the new weights' result, bit for bit."""
+import os
+import shutil
+import subprocess
+import sys
 import threading
 
 import numpy as np
@@ -98,3 +102,37 @@ def test_dropin_calls_from_several_threads(moehip):
     for t in threads:
         t.join()
     assert not wrong, wrong
+
+
+CHILD = """
+import ctypes, sys
+ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)   # its hipHostMalloc comes first
+import numpy as np
+import moehip, oracle as O
+assert not any(m.startswith("torch") for m in sys.modules)
+for dtype, M, N, K in ((2, 1, 768, 2048), (3, 8, 4000, 256)):
+    A = O.normal(M * K, 51, 0.0, 1.0).reshape(M, K)
+    w, s = (O.quant_q8 if dtype == 2 else O.quant_q4)(O.normal(N * K, 52, 0.0, 0.02).reshape(N, K))
+    for _ in range(3):
+        want = (O.gemv_q8 if dtype == 2 else O.gemv_q4)(A, w, s, N, K)
+        got = moehip.matmul_adaptive(A, None, {"q": w, "s": s, "dtype": dtype}, N, K)
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+        w.reshape(-1).view(np.uint8)[5] ^= 0x11
+assert ctypes.c_int.in_dll(ctypes.CDLL(sys.argv[1]), "refused").value > 0
+print("child ok")
+"""
+
+
+@pytest.mark.skipif(shutil.which("gcc") is None, reason="needs gcc for the refusing allocator")
+def test_dropin_without_pinned_memory(moehip, tmp_path):
+    """A host that refuses pinned memory: the drop-in takes its waiting copies,
+    as it did before it had a pinned staging."""
+    print("drop-in without pinned memory", flush=True)
+    src, so = tmp_path / "refuse.c", tmp_path / "refuse.so"
+    src.write_text("#include <stddef.h>\nint refused;\n"
+                   "int hipHostMalloc(void** p, size_t n, unsigned f) { (void)p; (void)n; (void)f; ++refused; return 2; }\n")
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(so), str(src)], check=True)
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    env = dict(os.environ, PYTHONPATH=os.pathsep.join([os.path.join(root, "moe.cc_amd"), os.path.join(root, "oracle")]))
+    r = subprocess.run([sys.executable, "-c", CHILD, str(so)], env=env, capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0 and "child ok" in r.stdout, r.stdout + r.stderr
