@@ -119,9 +119,12 @@ bool pin_staging() {
 }
 
 // 64-bit digest of a host buffer: eight lanes, each folding two 8-byte words
-// and its state through one 64 x 64 -> 128 bit product (16 bytes a multiply),
-// the lanes' old states kept beside the product so that a zero factor loses no
-// history; tail bytes folded in one at a time.
+// and its state through one 64 x 64 -> 128 bit product whose halves are XORed
+// (the mixing step of wyhash, Wang Yi; 16 bytes a multiply), the lanes' old
+// states kept beside the product so that a zero factor loses no history; tail
+// bytes folded in one at a time as FNV-1a does.  The keys are odd 64-bit
+// constants known from xxHash64, MurmurHash3's finaliser and wyhash; any well
+// mixed ones would do.
 uint64_t fold_product(uint64_t a, uint64_t b) {
   const unsigned __int128 p = (unsigned __int128)a * b;
   return (uint64_t)p ^ (uint64_t)(p >> 64);

@@ -1955,14 +1955,15 @@ moe_status dense_matmul(const DenseArgs& a, hipStream_t s) {
   if (a.pack_dtype && (!a.pack_part || !a.pack_tabs ||
                        !((a.sel_counter && dense_row_ok(a, vec)) || dense_rows4_ok(a, vec))))
     return set_error(MOE_ERR_ARG, "dense matmul: packing given rows needs the row kernel and the fused "
-                                  "selection, or the 5-16 token rows kernel");
+                                  "selection, or the 5-32 token rows kernel");
   if (dense_row_ok(a, vec)) {
     if (a.pack_dtype == 2) return launch_row<false, 2>(a, s);
     if (a.pack_dtype == 3) return launch_row<false, 3>(a, s);
     return launch_row<false, 0>(a, s);
   }
   if (dense_rows4_ok(a, vec) && !rows4_kernel_chosen()) {
-    // 5-16 given rows against few rows (the router): one block per row, one
+    // 5-32 given rows against few rows (the router): one block per row (and
+    // group of 16), one
     // consumer lane per token's sequential chain, three producer waves
     if (a.pack_dtype == 2) return launch_gemv<1, false, 2, 3, 16>(a, s);
     if (a.pack_dtype == 3) return launch_gemv<1, false, 3, 3, 16>(a, s);

@@ -303,9 +303,9 @@ __global__ __launch_bounds__(kBlock) void qgemv_fused(TiledArgs a) {
 // blocks, 25 so.)
 //
 // Bound: latency at a few MB (each block: its activations, two or three
-// dependent chunk loads, the reduction).  Q8 [1000 x 1030], 7 tokens: 20.2
-// us with one wave a row converting every activation per row, 7.9 us here;
-// [4096 x 4000], 64 tokens: 553 -> 37.
+// dependent chunk loads, the reduction).  Q8 [1000 x 1030], 7 tokens: 19.8
+// us with one wave a row converting every activation per row, 7.1 here (7.6
+// with one lane finishing a row's outputs); [4096 x 4000], 64 tokens: 553 -> 37.
 typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(1)));
 
 struct AnyArgs {

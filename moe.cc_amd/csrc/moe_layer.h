@@ -41,7 +41,7 @@ struct LayerDev {
   float* xn = nullptr;       // [T][D] normed input (block forward)
   uint32_t* hpart = nullptr; // [T*topk][h segments][2] partial headers of the h tables
   uint32_t* xpart = nullptr; // partial headers of the x tables packed by the router: up to 4
-                             // tokens [T][router blocks][2], 5-16 [router blocks][16][2]
+                             // tokens [T][router blocks][2], 5-32 [T / 16][router blocks][16][2]
   // grouped kernels: pairs per expert, first pair of each expert in `perm`,
   // pair ids (t * topk + j) grouped by expert, expert outputs per pair
   int* ecount = nullptr;     // [E]
