@@ -549,7 +549,8 @@ __global__ __launch_bounds__(kTileBlock) void gate_up_down_kernel(FuseArgs f) {
 // the first 2048 columns once (2048 columns, 5 tokens 5.8 -> 4.5 us with 256,
 // 512 tokens 6.9 -> 6.4).  Two such blocks fit a CU: past 512 rows they take a
 // second round, and 256 threads a row are better (2048 rows of 2048 columns
-// 19.2 -> 14.1, of 64 10.6 -> 5.7, of 1001 145 -> 69).
+// 19.2 -> 14.1, of 64 10.6 -> 5.7, of 1001 145 -> 29; 600 rows of 8192 columns,
+// whose squares leave room for few blocks either way, 27.6 -> 29.7).
 typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
 
 template <int NT>
@@ -1112,7 +1113,7 @@ static moe_status launch_rmsnorm(const float* x, const float* w, float* y, int T
 moe_status rmsnorm_dev(const float* x, const float* w, float* y, int T, int D, float eps) {
   if (T <= 0) return MOE_OK;
   const int fast = (D % 4 == 0) && aligned16(x) && (size_t)D * 4 <= kMaxLds;
-  if (T <= 512 && (D >= 512 || T < 256)) return launch_rmsnorm<512>(x, w, y, T, D, eps, fast);
+  if ((T <= 512 && (D >= 512 || T < 256)) || (T <= 768 && D > 6144)) return launch_rmsnorm<512>(x, w, y, T, D, eps, fast);
   return launch_rmsnorm<256>(x, w, y, T, D, eps, fast);
 }
 

@@ -303,10 +303,10 @@ def test_rmsnorm_dev(moehip):
 
 
 @pytest.mark.parametrize("T,D", [(255, 256), (256, 508), (256, 512), (512, 2052), (513, 4), (513, 2048), (600, 1001),
-                                 (520, 4100)])
+                                 (520, 4100), (514, 6148), (769, 6148)])
 def test_rmsnorm_many_rows(moehip, T, D):
-    """512 threads a row up to 512 rows, 256 past them and for many short
-    rows; odd lengths; the special rows of the sums among the others."""
+    """512 threads a row up to 512 rows (768 of very long ones), 256 past them
+    and for many short rows; odd lengths; the special rows of the sums among the others."""
     x = O.normal(T * D, 7 + D, 0.0, 2.0).reshape(T, D)
     n = min(D, 2048)
     x[T - 6:, :n] = _seq_sum_rows()[:, :n]
