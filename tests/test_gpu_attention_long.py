@@ -3,7 +3,7 @@
 every cached position), through the whole-model C ABI.
 
 The model tests in test_gpu_model.py stay inside one 64-key block.  These
-run the kernels' multi-block paths at configs[4]'s head geometry
+run the kernels' multi-block paths at the 30B-A3B model's head geometry
 (head_dim 128, 32 query heads, 4 KV heads) with small D and L:
 
 * a 320-token prompt in one chunk: the query-tiled score kernel over five
@@ -43,7 +43,7 @@ GEOM = dict(D=256, L=2, hd=128, nq=32, nkv=4, dff=128, E=16, V=300, dtype=3)
 
 
 def test_long_prompt_decode_and_second_chunk(moehip):
-    """configs[4]'s heads: 320-token prompt, 70 decode steps, a 70-token
+    """The 30B-A3B model's heads: 320-token prompt, 70 decode steps, a 70-token
     chunk at position 390, then forward_full of the whole sequence."""
     print("attention long: prompt 320 / decode 70 / chunk 70", flush=True)
     tm = O.TinyModel(seed=41, **GEOM)
